@@ -676,10 +676,14 @@ int vpa_chunked_prefill_paged_attention(
                 op, dtype_name(dtype), dtype_name(cache_dtype), head_dim, block_size);
   if (num_seqs == 0 || max_query_len == 0 || total_query_rows == 0) return VPA_OK;
   {
-    const int ppb = prefill_positions_per_workgroup(group);
+    // (the groups the MFMA kernel takes at run time keep the bound of the
+    // vector kernel, eight times the workgroups)
+    const bool fixed_group = group == 1 || group == 2 || group == 4;
+    const int64_t ppb = 128 / group;
     const int64_t grid =
-        mfma ? (int64_t)num_seqs * ((max_query_len + ppb - 1) / ppb) * (int64_t)num_kv_heads
-             : prefill_vector_workgroups(num_seqs, max_query_len, group, num_kv_heads);
+        mfma && fixed_group
+            ? (int64_t)num_seqs * (((int64_t)max_query_len + ppb - 1) / ppb) * (int64_t)num_kv_heads
+            : prefill_vector_workgroups(num_seqs, max_query_len, group, num_kv_heads);
     if (grid > ((int64_t)1 << 31) - 1)
       return fail(VPA_ERR_UNSUPPORTED, "%s: grid of %lld workgroups exceeds 2^31-1", op,
                   (long long)grid);

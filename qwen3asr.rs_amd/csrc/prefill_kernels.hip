@@ -126,6 +126,42 @@ __device__ __forceinline__ void dma16(const void* src, const void* lds) {
 template <int N>
 using Int = std::integral_constant<int, N>;
 
+// Two probabilities as two pairs of T each, high + low parts: high is p
+// rounded toward zero, so the low part is never negative, and it is kept
+// above zero wherever p is (well above T's smallest value): an infinite value
+// then adds +inf times a positive number twice, and the sum stays infinite
+// as it is with the f32 probability. f16 probabilities are scaled by
+// 2^kProbScaleLog2 (and with them the row sums), which moves f16's smallest
+// value to 2^-31 of a probability of 1; bf16 has f32's range.
+template <typename T>
+constexpr int kProbScaleLog2 = std::is_same_v<T, f16_t> ? 7 : 0;
+
+template <typename T>
+__device__ __forceinline__ uint32_t prob_high(float p0, float p1);
+template <>
+__device__ __forceinline__ uint32_t prob_high<bf16_t>(float p0, float p1) {
+  return (__float_as_uint(p1) & 0xffff0000u) | (__float_as_uint(p0) >> 16);
+}
+template <>
+__device__ __forceinline__ uint32_t prob_high<f16_t>(float p0, float p1) {
+  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(p0, p1));
+}
+template <typename T>
+__device__ __forceinline__ uint32_t prob_low(float p0, float p1, uint32_t high);
+template <>
+__device__ __forceinline__ uint32_t prob_low<bf16_t>(float p0, float p1, uint32_t high) {
+  // (the last bit set: the rest is at least 2^-24 of p)
+  return pack2_hw<bf16_t>(
+      __uint_as_float(__float_as_uint(p0) | 1u) - low_half_f32<bf16_t>(high),
+      __uint_as_float(__float_as_uint(p1) | 1u) - high_half_f32<bf16_t>(high));
+}
+template <>
+__device__ __forceinline__ uint32_t prob_low<f16_t>(float p0, float p1, uint32_t high) {
+  constexpr float kTiny = 5.9604645e-8f;  // 2^-24, f16's smallest value
+  return pack2_hw<f16_t>(fmaxf(p0 - low_half_f32<f16_t>(high), fminf(p0, kTiny)),
+                         fmaxf(p1 - high_half_f32<f16_t>(high), fminf(p1, kTiny)));
+}
+
 typedef int v4i_t __attribute__((ext_vector_type(4)));
 
 // LDS byte address of a __shared__ pointer.
@@ -256,6 +292,16 @@ constexpr int prefill_waves_per_eu() {
   return D > 128 ? 1 : VPA_PREFILL_WAVES_PER_EU;
 }
 
+// G: query heads per kv head (1, 2 or 4), or 0: any number of them, given at
+// run time (`group`). G = 0 enumerates the (position, head) rows of a kv head
+// heads-fastest, so a group that does not divide 32 still fills every row of
+// a wave, and keeps 16 (bf16) or 22 (f16) bits of each probability: P goes
+// through the P.V MFMAs as two values of T (prob_high, prob_low), half as
+// many MFMAs again, where the vector kernel kept P in f32. MFMA-bound like
+// the fixed groups. Measured with the append before it (f16, 32 query over
+// 4 kv heads, 12 sequences of 33-450 new over 0-700 prior tokens, 21.2
+// GFLOP): 58.7 us, against 766 us on the vector kernel; error against 64
+// bits 2.1e-4 both ways, the output's rounding.
 template <typename T, typename C, int D, int BS, int G>
 __global__ __launch_bounds__(kPrefillThreads)
 __attribute__((amdgpu_waves_per_eu(prefill_waves_per_eu<D>()))) void prefill_paged_kernel(
@@ -266,15 +312,16 @@ __attribute__((amdgpu_waves_per_eu(prefill_waves_per_eu<D>()))) void prefill_pag
     int32_t max_kv_len, int64_t total_query_rows, float scale_log2, float denom_eps,
     int32_t causal, int32_t num_heads, int32_t num_kv_heads, int64_t num_blocks,
     int64_t block_stride, int64_t head_stride, int32_t q_tiles, const float* __restrict__ k_scale,
-    const float* __restrict__ v_scale) {
+    const float* __restrict__ v_scale, int32_t group) {
   constexpr bool kF8 = std::is_same_v<C, fp8_t>;
   static_assert(kF8 || std::is_same_v<C, T>, "cache type is the query type or fp8");
   constexpr int KT = kPrefillKeys;
   constexpr int SUB = prefill_step_tiles<kF8, D, BS>();
   static_assert(SUB % kSoftmaxTiles == 0, "whole softmax groups per step");
   constexpr int X = kF8 ? 16 : 8;  // cache elements per 16-byte unit
-  constexpr int PPW = 32 / G;   // query positions per wave
-  constexpr int PPB = kPrefillWaves * PPW;  // query positions per workgroup
+  constexpr bool kAnyGroup = G == 0;
+  constexpr int PPW = kAnyGroup ? 32 : 32 / G;  // query positions per wave (G > 0)
+  constexpr int PPB = kPrefillWaves * PPW;      // query positions per workgroup (G > 0)
   constexpr int KS = D / 16;    // k-steps of Q.K^T
   constexpr int DT = D / 32;    // 32-row tiles of O^T
   // fp8 at 8-token blocks: a 16-byte value unit holds two dims (2r, 2r + 1)
@@ -339,10 +386,17 @@ __attribute__((amdgpu_waves_per_eu(prefill_waves_per_eu<D>()))) void prefill_pag
   else q_len = (int)min((int64_t)q_len, total_query_rows - (int64_t)qa);
   const int k_len = (int)min(ctx, (uint32_t)max_kv_len);
 
-  const int p0 = qt * PPB;
+  // first (position, head) row of this workgroup (kAnyGroup)
+  // (32 bits past the return: more rows than 2^32 do not fit the card)
+  if (kAnyGroup && (int64_t)qt * (kPrefillWaves * 32) >= (int64_t)q_len * group) return;
+  const uint32_t row0 = (uint32_t)qt * (kPrefillWaves * 32);
+  const uint32_t ugroup = (uint32_t)group;
+  const int p0 = kAnyGroup ? (int)(row0 / ugroup) : qt * PPB;
   if (p0 >= q_len) return;  // whole workgroup: tile past this sequence's queries
   const int shift = k_len - q_len;  // bottom-right causal alignment
-  const int wg_end = min(p0 + PPB, q_len);
+  const int wg_end =
+      kAnyGroup ? (int)min((row0 + kPrefillWaves * 32 - 1) / ugroup + 1, (uint32_t)q_len)
+                : min(p0 + PPB, q_len);
   const int n_keys = max(0, causal ? min(k_len, wg_end + shift) : k_len);
   const int n_tiles = (n_keys + KT - 1) / KT;
   const int n_steps = (n_tiles + SUB - 1) / SUB;
@@ -350,13 +404,17 @@ __attribute__((amdgpu_waves_per_eu(prefill_waves_per_eu<D>()))) void prefill_pag
   // this lane's query row (column of S^T and O^T)
   const int col = lane & 31;
   const int half = lane >> 5;
-  const int wpos0 = p0 + wave * PPW;
-  const int pos = wpos0 + col % PPW;
-  const int head = j * G + col / PPW;
+  const uint32_t wrow0 = row0 + wave * 32;  // (kAnyGroup)
+  const int wpos0 =
+      kAnyGroup ? (int)min(wrow0 / ugroup, (uint32_t)q_len) : p0 + wave * PPW;
+  const int pos =
+      kAnyGroup ? (int)min((wrow0 + col) / ugroup, (uint32_t)q_len) : wpos0 + col % PPW;
+  const int head = kAnyGroup ? j * group + (int)((wrow0 + col) % ugroup) : j * G + col / PPW;
   const bool row_ok = pos < q_len;
   const int64_t row = (int64_t)qa + pos;
   const int limit = causal ? pos + shift : k_len - 1;  // last key the row sees
-  const int wave_end = min(wpos0 + PPW, q_len);
+  const int wave_end = kAnyGroup ? (int)min((wrow0 + 31) / ugroup + 1, (uint32_t)q_len)
+                                 : min(wpos0 + PPW, q_len);
   const int wave_keys =
       wave_end <= wpos0 ? 0 : max(0, causal ? min(k_len, wave_end + shift) : k_len);
   const int wave_min_limit = causal ? wpos0 + shift : k_len - 1;
@@ -394,7 +452,8 @@ __attribute__((amdgpu_waves_per_eu(prefill_waves_per_eu<D>()))) void prefill_pag
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
     for (int e = 0; e < 16; ++e) o[dt][e] = 0.f;
-  const float sl = fabsf(scale_log2);
+  // (never 0: a masked score is -inf, and 0 * -inf would be NaN)
+  const float sl = fmaxf(fabsf(scale_log2), 1.17549435e-38f);
   float m = -INFINITY;   // reference max of the row (moves lazily), log2 units
   float mt = -INFINITY;  // the row's true max so far, log2 units
   float lsum = 0.f;      // this lane's share of the row's exp sum
@@ -611,12 +670,20 @@ __attribute__((amdgpu_waves_per_eu(prefill_waves_per_eu<D>()))) void prefill_pag
     for (int r = 1; r < 16; ++r) ps += sval[r];
     lsum += ps;
     uint4 pk[2];
+    uint4 pl[kAnyGroup ? 2 : 1];  // kAnyGroup: what pk left of the probabilities
 #pragma unroll
-    for (int k2 = 0; k2 < 2; ++k2)
-      pk[k2] = make_uint4(pack2_hw<T>(sval[8 * k2 + 0], sval[8 * k2 + 1]),
-                          pack2_hw<T>(sval[8 * k2 + 2], sval[8 * k2 + 3]),
-                          pack2_hw<T>(sval[8 * k2 + 4], sval[8 * k2 + 5]),
-                          pack2_hw<T>(sval[8 * k2 + 6], sval[8 * k2 + 7]));
+    for (int k2 = 0; k2 < 2; ++k2) {
+      const float* p = sval + 8 * k2;
+      if constexpr (kAnyGroup) {
+        pk[k2] = make_uint4(prob_high<T>(p[0], p[1]), prob_high<T>(p[2], p[3]),
+                            prob_high<T>(p[4], p[5]), prob_high<T>(p[6], p[7]));
+        pl[k2] = make_uint4(prob_low<T>(p[0], p[1], pk[k2].x), prob_low<T>(p[2], p[3], pk[k2].y),
+                            prob_low<T>(p[4], p[5], pk[k2].z), prob_low<T>(p[6], p[7], pk[k2].w));
+      } else {
+        pk[k2] = make_uint4(pack2_hw<T>(p[0], p[1]), pack2_hw<T>(p[2], p[3]),
+                            pack2_hw<T>(p[4], p[5]), pack2_hw<T>(p[6], p[7]));
+      }
+    }
     // k-step k2 of lane half h covers keys 16 k2 + 8h .. 16 k2 + 8h + 7, one
     // unit of row d = 32 dt + col (values of absent keys were zeroed in LDS
     // by the step)
@@ -640,6 +707,13 @@ __attribute__((amdgpu_waves_per_eu(prefill_waves_per_eu<D>()))) void prefill_pag
 #pragma unroll
       for (int k2 = 0; k2 < 2; ++k2)
         o[dt] = mfma32x32x16<T>(__builtin_bit_cast(uint4, vop[dt][k2]), pk[k2], o[dt]);
+    if constexpr (kAnyGroup) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int k2 = 0; k2 < 2; ++k2)
+          o[dt] = mfma32x32x16<T>(__builtin_bit_cast(uint4, vop[dt][k2]), pl[k2], o[dt]);
+    }
   };
 
   // the SUB tiles of step t in softmax groups of two: scores of both tiles
@@ -678,7 +752,9 @@ __attribute__((amdgpu_waves_per_eu(prefill_waves_per_eu<D>()))) void prefill_pag
           for (int e = 0; e < 16; ++e) o[dt][e] *= alpha;
         m = m_new;
       }
-      const float m_use = m == -INFINITY ? 0.f : m;  // a row without keys so far
+      // (0 for a row without keys so far; kAnyGroup scales f16 probabilities)
+      const float m_use =
+          (m == -INFINITY ? 0.f : m) - (kAnyGroup ? (float)kProbScaleLog2<T> : 0.f);
       accumulate(vst(sc, g0), sacc[0], m_use);
 #pragma unroll
       for (int u = 1; u < kSoftmaxTiles; ++u)
@@ -820,7 +896,8 @@ __attribute__((amdgpu_waves_per_eu(prefill_waves_per_eu<D>()))) void prefill_pag
   // larger
   const float total = sum_xor32(lsum);
   const float eps_m = denom_eps > 0.f && m != -INFINITY
-                          ? denom_eps * __builtin_amdgcn_exp2f(mt - m)
+                          ? denom_eps * __builtin_amdgcn_exp2f(
+                                            mt - m + (kAnyGroup ? kProbScaleLog2<T> : 0))
                           : 0.f;
   const float inv = total > 0.f ? vs / (total + eps_m) : 0.f;  // a row that sees no key gives 0
   if (row_ok) {
@@ -835,6 +912,12 @@ __attribute__((amdgpu_waves_per_eu(prefill_waves_per_eu<D>()))) void prefill_pag
                        pack2_hw<T>(o[dt][4 * i + 2] * inv, o[dt][4 * i + 3] * inv));
       }
   }
+}
+
+// Workgroups along the (position, head) rows of one (sequence, kv head).
+int64_t prefill_row_tiles(int32_t max_query_len, int32_t group) {
+  constexpr int kRows = kPrefillWaves * 32;
+  return ((int64_t)max_query_len * group + kRows - 1) / kRows;
 }
 
 // Arguments after the template dispatch, shared by every instance.
@@ -858,8 +941,8 @@ struct PrefillArgs {
 
 template <typename T, typename C, int D, int BS, int G>
 hipError_t launch_prefill_t(const PrefillArgs& a, const CacheGeom& g, hipStream_t stream) {
-  constexpr int kPositions = kPrefillWaves * 32 / G;
-  const int q_tiles = (a.max_query_len + kPositions - 1) / kPositions;
+  const int group = a.num_heads / g.num_kv_heads;
+  const int q_tiles = (int)prefill_row_tiles(a.max_query_len, group);
   const int64_t grid = (int64_t)a.num_seqs * q_tiles * g.num_kv_heads;
   if (grid == 0) return hipSuccess;
   const float scale_log2 = a.scale * 1.4426950408889634f;
@@ -871,7 +954,7 @@ hipError_t launch_prefill_t(const PrefillArgs& a, const CacheGeom& g, hipStream_
                      a.total_query_rows, scale_log2, a.denom_eps, a.causal, a.num_heads,
                      g.num_kv_heads,
                      g.num_blocks, g.block_stride, g.head_stride, q_tiles, a.k_scale,
-                     a.v_scale);
+                     a.v_scale, group);
   return hipGetLastError();
 }
 
@@ -886,7 +969,7 @@ hipError_t dispatch_group(int group, const PrefillArgs& a, const CacheGeom& g,
     case 4:
       return launch_prefill_t<T, C, D, BS, 4>(a, g, stream);
     default:
-      return hipErrorInvalidValue;
+      return launch_prefill_t<T, C, D, BS, 0>(a, g, stream);
   }
 }
 
@@ -939,15 +1022,12 @@ hipError_t dispatch_shape(int group, const PrefillArgs& a, const CacheGeom& g,
 }  // namespace
 
 bool prefill_supported(int dtype, int cache_dtype, int head_dim, int block_size, int group) {
-  if (!(dtype == VPA_DTYPE_BF16 || dtype == VPA_DTYPE_F16) || !(group == 1 || group == 2 ||
-                                                                group == 4))
-    return false;
+  if (!(dtype == VPA_DTYPE_BF16 || dtype == VPA_DTYPE_F16) || group < 1) return false;
   const bool fp8 = cache_dtype == VPA_DTYPE_FP8_E4M3;
   if (!fp8 && cache_dtype != dtype) return false;
   return prefill_shape(fp8, head_dim, block_size);
 }
 
-int prefill_positions_per_workgroup(int group) { return kPrefillWaves * 32 / group; }
 
 hipError_t launch_prefill_paged(int dtype, int cache_dtype, void* out, const void* query,
                                 const void* key_cache, const void* value_cache,

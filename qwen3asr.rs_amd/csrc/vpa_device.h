@@ -172,6 +172,28 @@ __device__ __forceinline__ uint32_t pack2_hw<f16_t>(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{lo, hi}, f16x2v_t));
 }
 
+// The low / high 16-bit element of a packed pair widened to f32 (exact).
+template <typename T>
+__device__ __forceinline__ float low_half_f32(uint32_t w);
+template <>
+__device__ __forceinline__ float low_half_f32<bf16_t>(uint32_t w) {
+  return __uint_as_float(w << 16);
+}
+template <>
+__device__ __forceinline__ float low_half_f32<f16_t>(uint32_t w) {
+  return f16_bits_to_f32((uint16_t)(w & 0xffffu));
+}
+template <typename T>
+__device__ __forceinline__ float high_half_f32(uint32_t w);
+template <>
+__device__ __forceinline__ float high_half_f32<bf16_t>(uint32_t w) {
+  return __uint_as_float(w & 0xffff0000u);
+}
+template <>
+__device__ __forceinline__ float high_half_f32<f16_t>(uint32_t w) {
+  return f16_bits_to_f32((uint16_t)(w >> 16));
+}
+
 // acc + a.lo*b.lo + a.hi*b.hi for two packed 16-bit pairs (v_dot2 on gfx950).
 template <typename T>
 __device__ __forceinline__ float dot2_acc(uint32_t a, uint32_t b, float acc);

@@ -202,8 +202,6 @@ hipError_t launch_prefill_vector(int dtype, int cache_dtype, void* out, const vo
                                  const float* k_scale, const float* v_scale,
                                  hipStream_t stream);
 
-// Query positions one prefill workgroup covers for a GQA group size.
-int prefill_positions_per_workgroup(int group);
 // True when the MFMA prefill kernel is compiled for this combination.
 bool prefill_supported(int dtype, int cache_dtype, int head_dim, int block_size, int group);
 

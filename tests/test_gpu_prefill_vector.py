@@ -136,3 +136,52 @@ def test_prefill_f32_row_without_keys_and_empty_sequences(device):
                             causal=False, mutate_bt=absent)
     assert_attention_close(got, want, orc.F32, "no keys")
     assert not np.any(got[5:12])
+
+
+@pytest.mark.parametrize("code", [orc.BF16, orc.F16])
+@pytest.mark.parametrize("group,kvh,d,bs,fp8", [(3, 8, 128, 16, False), (5, 1, 64, 32, False),
+                                                (7, 2, 192, 8, False), (48, 1, 96, 16, False),
+                                                (130, 1, 64, 16, True), (8, 2, 256, 32, True)])
+def test_prefill_any_group_keeps_f32_probabilities(device, code, group, kvh, d, bs, fp8):
+    """16-bit queries with any number of query heads per kv head on the MFMA
+    kernel: (position, head) row tiles of 128 rows that end inside a position
+    (groups that divide neither 32 nor 128, and one above 128), 1 to 129 new
+    tokens. The probabilities keep more than 16 bits: next to the output's
+    own rounding (half a unit in the last place, at most 2^-8 of the value in
+    bf16 and 2^-11 in f16) an element may be off by what the probabilities'
+    two parts leave (2^-17 in bf16, whose parts hold 16 bits; 2^-20 covers
+    f16's 22 bits and the f32 sums) times the largest |value| behind it
+    (below 12 here: 6 standard deviations times the fp8 data's 2)."""
+    got, want = vector_case(device, code, group * kvh, kvh, d, bs, [0, 37, 300, 1], [1, 43, 129, 2],
+                            seed=group + d, causal=True, fp8=fp8)
+    half, low = (2.0 ** -8, 2.0 ** -17) if code == orc.BF16 else (2.0 ** -11, 2.0 ** -20)
+    err = np.abs(got.astype(np.float64) - want)
+    bound = half * np.abs(want) + 12 * low
+    assert np.all(np.isfinite(got))
+    assert np.max(err / bound) <= 1.0, f"worst {np.max(err / bound):.2f} of the bound"
+
+
+@pytest.mark.parametrize("code", [orc.BF16, orc.F16])
+def test_prefill_any_group_infinite_values_and_zero_scale(device, code):
+    """An infinite cached value gives an infinite output (not NaN) in the rows
+    that see it, and a softmax scale of 0 the mean of the visible values."""
+    h, kvh, d, bs, n = 6, 2, 64, 16, 40
+    rng = np.random.default_rng(3)
+    kc, vc = make_cache(rng, 4, kvh, d, bs, code)
+    vc = orc.to_f32(vc, code).astype(np.float32)
+    vc[1, 1, 5, 3] = np.inf  # head 1, dim 5, token 3
+    vc = orc.from_f32(vc, code)
+    bt = np.array([[1, 2, 3]], dtype=np.uint32)
+    q = random_words(rng, (n, h, d), code)
+    args = (to_dev(q, code, device), to_dev(kc, code, device), to_dev(vc, code, device),
+            u32(bt, device), u32([n], device), u32([0, n], device), None, None)
+    out = vpa.paged_attention_varlen_prefill(*args, d ** -0.5, 1.0, causal=False)
+    got = orc.to_f32(to_host(out), code)
+    assert np.all(np.isposinf(got[:, 3:, 5]))
+    got[:, 3:, 5] = 0
+    assert np.all(np.isfinite(got))
+    out = vpa.paged_attention_varlen_prefill(*args, 0.0, 1.0, causal=True)
+    got = orc.to_f32(to_host(out), code)[:, :3]
+    v = orc.to_f32(vc, code)[1:, 0].transpose(0, 2, 1).reshape(-1, d)[:n]
+    want = np.cumsum(v.astype(np.float64), axis=0) / np.arange(1, n + 1)[:, None]
+    assert_attention_close(got, np.repeat(want[:, None], 3, axis=1), code, "scale 0")
