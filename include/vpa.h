@@ -389,11 +389,11 @@ int vpa_gather_kv_cache(void* out_key, void* out_value, const void* key_cache,
  * Head dims 64, 96, 128, 192 and 256 (the Metal kernel's set,
  * varlen_prefill.rs:15), block_size 8, 16 or 32, any number of query heads
  * per kv head; cache_dtype equals dtype or is VPA_DTYPE_FP8_E4M3 (for any
- * query type). bf16 / f16 queries with 1, 2 or 4 query heads per kv head
- * run on the MFMA kernel where a (block, head) tile is a whole number of
- * 1 KiB DMAs (head_dim 96 at 16- or 32-token blocks for 16 bits, 32-token
- * blocks for fp8; fp8 at 8-token blocks head_dim 128 or 256); every other
- * configuration, f32 included, on a vector-ALU kernel with f32 arithmetic.
+ * query type). bf16 / f16 queries run on the 16-bit MFMA kernel where a
+ * (block, head) tile is a whole number of 1 KiB DMAs (head_dim 96 at 16- or
+ * 32-token blocks for 16 bits, 32-token blocks for fp8; fp8 at 8-token blocks
+ * head_dim 128 or 256) and on a vector-ALU kernel with f32 arithmetic at the
+ * other shapes; f32 queries run on the f32 matrix instructions.
  * An fp8 cache is read as byte * k_scale / byte * v_scale (the Metal
  * kernel's fp8 path, prefill_paged_attn.metal:698-769, 797-800), converted
  * to the query type. Needs no workspace; safe under stream capture.

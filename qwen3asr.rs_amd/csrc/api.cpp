@@ -701,7 +701,9 @@ int vpa_chunked_prefill_paged_attention(
                 block_table_stride, max_kv_len, block_size);
   CacheGeom g{num_kv_heads, head_dim, block_size, num_blocks, cache_block_stride,
               cache_head_stride};
-  const auto launch = mfma ? launch_prefill_paged : launch_prefill_vector;
+  const auto launch = mfma                     ? launch_prefill_paged
+                      : dtype == VPA_DTYPE_F32 ? launch_prefill_f32
+                                               : launch_prefill_vector;
   return hip_status(op, launch(dtype, cache_dtype, out, query, key_cache, value_cache,
                                block_tables, block_table_stride, cu_seqlens_q, context_lens,
                                num_seqs, max_query_len, max_kv_len, total_query_rows,

@@ -1,16 +1,15 @@
 // Chunked-prefill attention over the paged cache on the vector ALUs: the
-// configurations the MFMA kernel (prefill_kernels.hip) does not take. f32
-// queries over f32 or fp8 caches (the Metal prefill's `float` and
-// `float, uint8_t` instances, vasr-paged-attn/src/metal/kernels/
-// prefill_paged_attn.metal:1606, 1610, dispatched for F32 at
-// vasr-paged-attn/src/metal/kernels/mod.rs:119-137), any number of query
-// heads per kv head (the Metal dispatch takes q_per_kv as a grid dimension,
-// mod.rs:145-283), and the 16-bit head-dim / block-size pairs without a
-// whole number of 1 KiB DMAs per tile.
+// configurations the matrix-core kernels (prefill_kernels.hip,
+// prefill_f32_kernels.hip) do not take, which are 16-bit queries at the
+// head-dim / block-size pairs without a whole number of 1 KiB DMAs per tile,
+// with any number of query heads per kv head (the Metal dispatch takes
+// q_per_kv as a grid dimension, vasr-paged-attn/src/metal/kernels/
+// mod.rs:145-283).
 //
 // Decode (paged_attention) runs the head-dim / block-size pairs its own
-// kernels do not take on this kernel too, with one query per sequence (no
-// cu_seqlens_q), causal, over the whole context, and denom_eps 1e-6.
+// kernels do not take on this kernel too, f32 queries over fp8 caches among
+// them, with one query per sequence (no cu_seqlens_q), causal, over the
+// whole context, and denom_eps 1e-6.
 //
 // Semantics are the MFMA kernel's: query i of a sequence with n queries and
 // L keys sees keys t <= i + L - n when causal (bottom-right alignment, the
@@ -36,9 +35,9 @@
 // no f32 rounding chain is longer than a quarter of the head dim or one
 // tile's keys (at head dim 256 a single running sum put elements near zero
 // past the f32 bound against the fp64 oracle).
-// Measured on c4's lengths with 24 query heads (3 per kv head): 14.6 ms in
-// f32, 13.3 ms in bf16 (23-25 TFLOP/s); the MFMA kernel runs the bf16 c4
-// shape at ~310 us.
+// Measured at head dim 128 on c4's lengths with 24 query heads (3 per kv
+// head): 13.3 ms in bf16 (25 TFLOP/s); the MFMA kernel runs the bf16 c4 shape
+// at ~310 us.
 #include <type_traits>
 
 #include "vpa_device.h"
@@ -398,7 +397,8 @@ hipError_t launch_prefill_vector(int dtype, int cache_dtype, void* out, const vo
       cu_seqlens_q, context_lens, num_seqs, max_query_len, max_kv_len, total_query_rows, scale, \
       denom_eps, causal, num_heads, g, k_scale, v_scale, stream
   if (dtype == VPA_DTYPE_F32)
-    return f8 ? vector_dim<float, fp8_t>(VPA_VEC_ARGS) : vector_dim<float, float>(VPA_VEC_ARGS);
+    // (f32 caches: prefill_f32_kernels.hip, and every decode shape has a kernel)
+    return f8 ? vector_dim<float, fp8_t>(VPA_VEC_ARGS) : hipErrorInvalidValue;
   if (dtype == VPA_DTYPE_BF16)
     return f8 ? vector_dim<bf16_t, fp8_t>(VPA_VEC_ARGS)
               : vector_dim<bf16_t, bf16_t>(VPA_VEC_ARGS);

@@ -184,11 +184,22 @@ hipError_t launch_prefill_paged(int dtype, int cache_dtype, void* out, const voi
                                 const float* k_scale, const float* v_scale,
                                 hipStream_t stream);
 
-// The vector-ALU prefill (prefill_vector_kernels.hip): f32 queries over f32
-// or fp8 caches, any number of query heads per kv head, and the 16-bit
-// shapes the MFMA kernel does not take; also the decode of the head-dim /
-// block-size pairs no decode kernel takes (cu_seqlens_q null: one query per
-// sequence). Same arguments as launch_prefill_paged.
+// The f32 prefill on the f32 matrix instructions (prefill_f32_kernels.hip):
+// f32 queries over f32 or fp8 caches, every shape. Same arguments.
+hipError_t launch_prefill_f32(int dtype, int cache_dtype, void* out, const void* query,
+                              const void* key_cache, const void* value_cache,
+                              const uint32_t* block_tables, int32_t block_table_stride,
+                              const uint32_t* cu_seqlens_q, const uint32_t* context_lens,
+                              int32_t num_seqs, int32_t max_query_len, int32_t max_kv_len,
+                              int64_t total_query_rows, float scale, float denom_eps,
+                              int32_t causal, int32_t num_heads, const CacheGeom& g,
+                              const float* k_scale, const float* v_scale, hipStream_t stream);
+
+// The vector-ALU prefill (prefill_vector_kernels.hip): the 16-bit shapes the
+// MFMA kernel does not take; also the decode of the head-dim / block-size
+// pairs no decode kernel takes (cu_seqlens_q null: one query per sequence).
+// Same arguments as launch_prefill_paged. (prefill_vector_supported names
+// the whole set, f32 prefills included, which launch_prefill_f32 serves.)
 bool prefill_vector_supported(int dtype, int cache_dtype, int head_dim, int block_size);
 int64_t prefill_vector_workgroups(int32_t num_seqs, int32_t max_query_len, int32_t group,
                                   int32_t num_kv_heads);

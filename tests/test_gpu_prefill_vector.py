@@ -185,3 +185,18 @@ def test_prefill_any_group_infinite_values_and_zero_scale(device, code):
     v = orc.to_f32(vc, code)[1:, 0].transpose(0, 2, 1).reshape(-1, d)[:n]
     want = np.cumsum(v.astype(np.float64), axis=0) / np.arange(1, n + 1)[:, None]
     assert_attention_close(got, np.repeat(want[:, None], 3, axis=1), code, "scale 0")
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("d,bs,n,prior", [(128, 16, 31, 70), (64, 32, 33, 5), (96, 8, 64, 129)])
+def test_prefill_f32_many_short_rows(device, d, bs, n, prior, fp8):
+    """Many row tiles over at most 320 keys: a wave of the f32 kernel takes a
+    row tile of its own instead of a quarter of one tile's keys (the other
+    cases here have fewer than 1024 tiles, and split)."""
+    if fp8 and bs == 8:
+        bs = 16
+    b = 129
+    rng = np.random.default_rng(n)
+    got, want = vector_case(device, orc.F32, 8, 8, d, bs, rng.integers(0, prior + 1, b),
+                            rng.integers(1, n + 1, b), seed=d + n, fp8=fp8)
+    assert_attention_close(got, want, orc.F32, f"d={d} bs={bs} fp8={fp8}")
