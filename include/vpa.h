@@ -186,7 +186,9 @@ int vpa_paged_attention(void* out, const void* query, const float* k_scale,
  * is per-step metadata like them). Arguments mean what they mean in
  * vpa_paged_attention (dtype: the query type; the list is the same for
  * every cache type); the workspace is that call's. Stream-ordered and
- * capture-safe; a no-op for configurations whose kernel needs no list.
+ * capture-safe; a no-op for configurations whose kernel never takes a list
+ * (decodes of few sequences work their items out themselves; the list is
+ * written for them too, for paged_cache_read).
  * No counterpart in the reference (its decode kernel sizes its grid from
  * max_context_len only).
  */
@@ -283,10 +285,12 @@ int vpa_reshape_and_cache_paged_attention_planned(
  * device array of the library, 64 MiB per GPU (build-time
  * VPA_NOALLOC_SCRATCH_MIB; `make NOALLOC_SCRATCH_MIB=<n>`), held until the
  * process ends by every process that loads the library, whether or not it
- * calls this entry point, and laid out for the kernel this configuration runs (16-bit / fp8 caches
- * on the rows kernel: num_seqs * num_heads * ceil(max_context_len / 2048)
- * partial rows of (head_dim + 32) floats, 5.3 MB at batch 256 / context
- * 4096, 42 MB at batch 1024 / context 8192). A call whose layout does not
+ * calls this entry point, and laid out as a caller's workspace where that
+ * fits, else for the longest partitions the kernel of this configuration
+ * takes (16-bit / fp8 caches on the rows kernel: num_seqs * num_heads *
+ * ceil(max_context_len / 2048) partial rows of (head_dim + 32) floats, 5.3 MB
+ * at batch 256 / context 4096, 42 MB at batch 1024 / context 8192). A call
+ * whose layout does not
  * fit returns VPA_ERR_WORKSPACE (after the other argument checks, before
  * touching the device). Same arguments (minus the workspace), results and
  * errors as vpa_paged_attention. Every call on a GPU shares that GPU's

@@ -342,11 +342,15 @@ int paged_attention_impl(void* out, const void* query, const float* k_scale,
         (append->key_token_stride * eb) % 16 != 0 || (append->value_token_stride * eb) % 16 != 0)
       return fail(VPA_ERR_INVALID_ARGUMENT, "%s: key/value rows must be 16-byte aligned", op);
   }
-  const int part_tokens =
-      scratch != nullptr ? decode_part_tokens(dtype, head_dim, block_size)
-                         : kDecodeMinPartitionTokens;
-  const size_t need =
+  // (the library's scratch is laid out like a caller's workspace where that
+  // fits it, else for the partition of the kernel that runs)
+  int part_tokens = kDecodeMinPartitionTokens;
+  size_t need =
       decode_workspace_bytes(num_seqs, num_heads, head_dim, max_context_len, part_tokens);
+  if (scratch != nullptr && need > scratch->bytes) {
+    part_tokens = decode_part_tokens(dtype, head_dim, block_size);
+    need = decode_workspace_bytes(num_seqs, num_heads, head_dim, max_context_len, part_tokens);
+  }
   if (scratch != nullptr) {
     if (need > scratch->bytes)
       return fail(VPA_ERR_WORKSPACE,
@@ -536,7 +540,7 @@ int vpa_paged_attention_plan(const uint32_t* context_lens, int32_t max_context_l
                 workspace == nullptr ? (size_t)0 : workspace_bytes);
   if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0)
     return fail(VPA_ERR_INVALID_ARGUMENT, "%s: workspace must be 256-byte aligned", op);
-  CacheGeom g{num_kv_heads, head_dim, block_size, 1, 0, 0};
+  CacheGeom g{num_kv_heads, head_dim, block_size, 1, 0, 0, decode_kv_rep(num_heads, num_kv_heads)};
   DecodeWorkspace ws =
       carve_decode_workspace(workspace, num_seqs, num_heads, head_dim, max_context_len);
   return hip_status(op, launch_decode_plan(dtype, context_lens, max_context_len,
@@ -581,7 +585,7 @@ int vpa_paged_cache_read(const void* key_cache, const void* value_cache,
   if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0)
     return fail(VPA_ERR_INVALID_ARGUMENT, "%s: workspace must be 256-byte aligned", op);
   CacheGeom g{num_kv_heads, head_dim, block_size, num_blocks, cache_block_stride,
-              cache_head_stride};
+              cache_head_stride, decode_kv_rep(num_heads, num_kv_heads)};
   const DecodeWorkspace ws =
       carve_decode_workspace(workspace, num_seqs, num_heads, head_dim, max_context_len);
   return hip_status(op, launch_paged_read(cache_dtype, key_cache, value_cache, block_tables,

@@ -4,7 +4,10 @@
 //     them: a work list built on the device (decode_plan_kernel, longest
 //     chunk first), paged_decode_rows_kernel (one workgroup per (chunk, kv
 //     head), its waves splitting the chunk's blocks) and decode_merge_kernel
-//     for the sequences longer than one chunk; described further down;
+//     for the sequences longer than one chunk; described further down. The
+//     rows kernel is in decode_rows.h; at most 64 sequences of at most 512
+//     tokens, or 128 (sequence, kv head) pairs, run its form without a work
+//     list (decode_small_kernels.hip);
 //   * f32 caches, fp8 caches under f32 queries, and the 16-bit / fp8 tiles
 //     above 8 KiB (head dims 192 and 256 at 32-token blocks):
 //     paged_decode_kernel, one wavefront per (kv head, sequence, split-K
@@ -43,6 +46,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "decode_rows.h"
 #include "vpa_device.h"
 #include "vpa_internal.h"
 
@@ -50,41 +54,6 @@ namespace vpa {
 namespace {
 
 constexpr int kPT = kDecodePartitionTokens;
-
-#ifndef VPA_DECODE_STREAM_LOADS
-#define VPA_DECODE_STREAM_LOADS 1
-#endif
-// K/V tile loads of the decode: every byte is read once per call, so they
-// stream (non-temporal) unless VPA_DECODE_STREAM_LOADS is 0.
-__device__ __forceinline__ uint4 tile_load(const uint4* p) {
-  if constexpr (VPA_DECODE_STREAM_LOADS) return load_stream(p);
-  else return *p;
-}
-// Workgroup barrier for data exchanged through LDS: waits for this wave's LDS
-// operations only (outstanding global loads and stores stay in flight).
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-// v with its 16-bit element e (0..7; uniform) replaced by val, without a
-// runtime-indexed array
-__device__ __forceinline__ uint4 put_u16(uint4 v, int e, uint32_t val) {
-  const uint32_t sh = (uint32_t)(e & 1) * 16u;
-  const uint32_t keep = ~(0xffffu << sh), ins = (val & 0xffffu) << sh;
-  const int w = e >> 1;
-  v.x = w == 0 ? (v.x & keep) | ins : v.x;
-  v.y = w == 1 ? (v.y & keep) | ins : v.y;
-  v.z = w == 2 ? (v.z & keep) | ins : v.z;
-  v.w = w == 3 ? (v.w & keep) | ins : v.w;
-  return v;
-}
-// 16-byte non-temporal store (the fused append's whole sectors)
-__device__ __forceinline__ void tile_store(uint4* p, const uint4& v) {
-  typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-  __builtin_nontemporal_store(u32x4{v.x, v.y, v.z, v.w}, reinterpret_cast<u32x4*>(p));
-}
 
 // E4M3FN byte b (0..255) of an fp8 cache as f32 (exact, through gfx950's
 // conversion to bf16)
@@ -455,8 +424,8 @@ __global__ __launch_bounds__(64) void paged_decode_kernel(
 // whose (block, head) tiles are whole 1 KiB wave loads of at most 8 KiB).
 //
 // Work list: decode_plan_kernel (one workgroup) turns context_lens into the
-// list of (sequence, chunk) items, longest first, a chunk being NW * PT
-// tokens, and a small header {0, item count}. All of it lives in the caller's
+// list of (sequence, chunk) items, longest first, a chunk being at most NW *
+// PT tokens (list_chunk), and a small header {log2 of the chunk, item count}. All of it lives in the caller's
 // workspace and is rebuilt by every call, so the launches can be captured
 // in a graph and replayed with new lengths; max_context_len only sizes the
 // grid, surplus workgroups exit at once.
@@ -487,15 +456,6 @@ __global__ __launch_bounds__(64) void paged_decode_kernel(
 // measured with only that fence added, c3 decode went from 176 to 823 us
 // per layer, against 4.7 us for the extra launch.)
 // ---------------------------------------------------------------------------
-// Floats per split-K partial row of the rows path: D outputs + a 32-float
-// line holding {max, sum}.
-template <int D>
-constexpr int kPartRow = D + 32;
-
-__device__ __forceinline__ int clamp_context(uint32_t ctx, int max_ctx, int cap) {
-  return min((int)min(ctx, (uint32_t)max_ctx), cap);
-}
-
 // Items are emitted longest first: a counting sort over kPlanBuckets
 // classes of chunk length, stable within a class, so full chunks start
 // first and the last workgroups the dispatcher hands out are short, which
@@ -576,7 +536,7 @@ __global__ __launch_bounds__(1024) void decode_plan_kernel(
     }
   }
   if (tid == 0) {
-    queue[0] = 0u;
+    queue[0] = (uint32_t)__builtin_ctz((unsigned)part_tokens);
     queue[1] = s_base[NB];
   }
 }
@@ -584,523 +544,6 @@ __global__ __launch_bounds__(1024) void decode_plan_kernel(
 #ifndef VPA_DECODE_MERGE_WAVES_PER_CU
 #define VPA_DECODE_MERGE_WAVES_PER_CU 16
 #endif
-#ifndef VPA_DECODE_NV
-#define VPA_DECODE_NV 8
-#endif
-#ifndef VPA_DECODE_FP8_NV
-#define VPA_DECODE_FP8_NV 4
-#endif
-#ifndef VPA_DECODE_ROWS_WAVES_PER_EU
-#define VPA_DECODE_ROWS_WAVES_PER_EU 3
-#endif
-
-// Workgroup of NW waves = one (sequence, kv head, chunk of NW * PT tokens)
-// work unit. Wave w attends over partition w of the chunk (PT tokens); the NW
-// partial results are merged in LDS, so HBM partial rows are only written for
-// sequences longer than one chunk.
-//
-// C is the cache element type: T itself, or fp8_t (E4M3FN bytes, 16 per
-// vector). With fp8 each 16-byte K or V vector is converted once to two
-// vectors of T (exact, v_cvt_scalef32_pk_*_fp8 with scale 1) and the same
-// v_dot2 products follow; a lane's q chunk is then 16 dims (two vectors),
-// *k_scale is folded into the softmax scale and *v_scale into the output.
-// Waves per SIMD the rows kernel is compiled for: instances with many q
-// vectors per lane (16-byte vectors: G x chunks per lane, two per chunk for
-// fp8) would spill at 3 (with 512-token waves: 16 and more).
-#ifndef VPA_DECODE_FP8_WAVES_PER_EU
-#define VPA_DECODE_FP8_WAVES_PER_EU VPA_DECODE_ROWS_WAVES_PER_EU
-#endif
-template <typename C, int D, int BS, int G>
-constexpr int rows_waves_per_eu() {
-  constexpr bool f8 = sizeof(C) == 1;
-  constexpr int qvec = G * (D * BS / ((f8 ? 16 : 8) * 64)) * (f8 ? 2 : 1);
-  return qvec >= 16 ? 2 : f8 ? VPA_DECODE_FP8_WAVES_PER_EU : VPA_DECODE_ROWS_WAVES_PER_EU;
-}
-
-// kAppend (16-bit caches): the launch also appends each sequence's new K/V
-// row (new_key / new_value, one token per sequence) at position L - 1 of its
-// context, the slot vASR's decode metadata gives the step's token
-// (paged_kv_cache.rs:985-1017), in place of a reshape_and_cache launch before
-// it. The wave whose partition ends at the context's last block holds that
-// block's K and V tiles in registers anyway: it stages the two new rows in
-// LDS at its start, puts the token's values into the tiles before using
-// them, and writes back whole 32-byte sectors with non-temporal stores: the
-// 16 key units of the token with their neighbours (tokens 2i, 2i + 1 share a
-// sector), and the whole value tile (every 32-byte value row holds the
-// token). No partially written sector reaches HBM.
-template <typename T, typename C, int D, int BS, int G, int PT, int NW, bool kAppend = false>
-__global__ __launch_bounds__(64 * NW)
-__attribute__((amdgpu_waves_per_eu(rows_waves_per_eu<C, D, BS, G>())))
-void paged_decode_rows_kernel(
-    T* __restrict__ out, const T* __restrict__ query, const C* __restrict__ key_cache,
-    const C* __restrict__ value_cache, const uint32_t* __restrict__ block_tables,
-    int32_t block_table_stride, float scale, int32_t num_heads, int32_t num_kv_heads,
-    int64_t num_blocks, int64_t block_stride, int64_t head_stride, float* __restrict__ part_out,
-    int32_t max_parts, const uint2* __restrict__ items, const uint32_t* __restrict__ queue,
-    int32_t num_seqs, int32_t max_ctx, int32_t cap_tokens, const float* __restrict__ k_scale,
-    const float* __restrict__ v_scale, const T* __restrict__ new_key,
-    const T* __restrict__ new_value, int64_t new_key_stride, int64_t new_value_stride,
-    int32_t kv_rep) {
-  constexpr bool kF8 = std::is_same_v<C, fp8_t>;
-  static_assert(kF8 || std::is_same_v<C, T>, "cache type is the query type or fp8");
-  static_assert(!(kAppend && kF8), "the fused append writes 16-bit caches");
-  constexpr int X = pack_x<C>();
-  static_assert(X == (kF8 ? 16 : 8), "16-bit or fp8 cache elements only");
-  constexpr int PB = PT / BS;        // blocks per wave partition
-  // fp8 at 8-token blocks: a 16-byte value vector holds two rows (dims 2r
-  // and 2r + 1) of the block's 8 tokens; otherwise VPR vectors make a row.
-  constexpr bool kPairRows = kF8 && BS == 8;
-  constexpr int VPR = kPairRows ? 1 : BS / X;  // 16-byte vectors per value row
-  constexpr int NVV = D * BS / X / 64;          // value vectors per lane per block
-  constexpr int NACC = kPairRows ? 2 * NVV : NVV;  // value rows per lane
-  constexpr int DSTEP = 64 / VPR;    // row stride between a lane's value vectors
-  constexpr int NPL = PT / 64;       // partition tokens per lane in the softmax
-  // Stages of NV loads per lane: 8 (8 KiB per wave) for 16-bit caches, 4
-  // for fp8, whose stages of 8 hold twice the tokens and twice the
-  // conversion and dot-product work between loads (measured: 4 loads per
-  // stage 3-5 % faster on fp8 c3 than 8). A K stage reads BKS
-  // key tiles: load k of a tile gives lane l vector l + 64k, i.e. token
-  // l % BS and 16-byte chunk l / BS + k * (64 / BS), so each instruction
-  // reads 1 KiB contiguous and the lane needs only those chunks of q
-  // (held in registers); the partial dot products of a token are summed
-  // over its 64 / BS lanes with DPP / permlane swaps. A V stage reads BKS
-  // value tiles the same way (lane l: row l / (BS/8) + k * 64 / (BS/8),
-  // tokens (l % (BS/8)) * 8 .. +7).
-  constexpr int KPL = D * BS / (X * 64);  // loads per lane per tile (K or V)
-  // 16-byte loads per lane per stage: the whole tiles that fit NV0 loads,
-  // at least one tile (head dims 96 and 192 give 3 or 6 loads per tile)
-  constexpr int NV0 = kF8 ? VPA_DECODE_FP8_NV : VPA_DECODE_NV;
-  constexpr int NV = KPL >= NV0 ? KPL : (NV0 / KPL) * KPL;
-  constexpr int LPT = 64 / BS;            // lanes per token in a key tile
-  constexpr int BKS = NV / KPL;           // tiles per stage
-  static_assert(KPL == NVV && KPL >= 1 && KPL <= NV && NV % KPL == 0, "stage shape");
-  static_assert(VPR >= 1 && VPR <= 4 && PB <= 64 && PT % 64 == 0 && PT >= D, "shape");
-
-  __shared__ float s_logit[NW][G][PT];
-  __shared__ __align__(16) uint16_t s_p[NW][G][PT];
-  __shared__ float s_m[NW][G], s_l[NW][G];
-  constexpr int NR = D / 8;  // 16-byte vectors of a new 16-bit K (or V) row
-  __shared__ __align__(16) uint4 s_new[kAppend ? 2 * NR : 1];
-
-  const int lane = threadIdx.x & 63;
-  // Uniform where a stage holds at most two tiles: the partition bounds,
-  // block ids and tile addresses derived from the wave index then stay in
-  // scalar registers (with more tiles per stage their addresses would not
-  // fit them and spill).
-  const int wave = BKS <= 2 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)
-                            : (int)(threadIdx.x >> 6);
-  const uint32_t w = blockIdx.x;
-  const int j = (int)(w % (uint32_t)num_kv_heads);
-  const uint32_t want = w / (uint32_t)num_kv_heads;  // index of this workgroup's item
-  // the list holds num_seqs * ceil(max_ctx / 128) >= gridDim.x / num_kv_heads
-  // entries, so the item is read together with the count (one round trip)
-  const uint32_t nitems = queue[1];
-  const uint2 item = items[want];
-  // (the empty asm keeps the compiler from sinking the item load below the
-  // count test)
-  asm volatile("" ::"s"(nitems), "s"(item.x), "s"(item.y));
-  if (want >= nitems) return;  // surplus workgroup of the grid
-  const int s = (int)(item.x >> 16);
-  const int chunk = (int)(item.x & 0xffffu);
-  // a work list built by an earlier call is only trusted within this call's
-  // bounds (sequence index, context cap), so every access stays in range
-  if (s >= num_seqs) return;
-  const int L = clamp_context(item.y, max_ctx, cap_tokens);
-  if (L <= 0) {
-    if (chunk == 0)
-      for (int i = threadIdx.x; i < G * D; i += 64 * NW)
-        store_from_f32<T>(out + ((int64_t)s * num_heads + j * G) * D + i, 0.f);
-    return;
-  }
-  const int nblk = (L + BS - 1) / BS;
-  const int nchunks = (nblk + PB * NW - 1) / (PB * NW);
-  // an item past the sequence's chunks (a list built for other lengths or
-  // another max_context_len) would write a partial row outside (s, h) or
-  // race with chunk 0 on the output: skip it
-  if (chunk >= nchunks || chunk >= max_parts) return;
-  // the chunk's blocks are split evenly over the NW waves (at most PB each),
-  // so short sequences keep every wave busy
-  const int c_begin = chunk * PB * NW;
-  const int c_nb = min(PB * NW, nblk - c_begin);
-  const int b_begin = c_begin + (c_nb * wave) / NW;
-  const int nb = c_begin + (c_nb * (wave + 1)) / NW - b_begin;  // 0: idle wave
-  // fused append: this wave's partition ends at the context's last block,
-  // which holds the new token at offset app_off (a context clamped by
-  // max_context_len or the table appends nothing)
-  const bool app = kAppend && nb > 0 && b_begin + nb == nblk && item.y == (uint32_t)L;
-  const int app_off = (L - 1) % BS;
-
-  float acc[G][NACC];
-  float m[G], lsum[G];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    m[g] = -INFINITY;
-    lsum[g] = 0.f;
-#pragma unroll
-    for (int k = 0; k < NACC; ++k) acc[g][k] = 0.f;
-  }
-
-  float vs = 1.f;  // value scale of an fp8 cache
-  if constexpr (kF8) {
-    scale *= *k_scale;
-    vs = *v_scale;
-  }
-  // logits are kept in log2 units (scale * log2 e folded in), so every
-  // exponential below is one v_exp_f32; the partial rows' maxima are in the
-  // same units for decode_merge_kernel
-  scale *= 1.4426950408889634f;
-
-  if (nb > 0) {
-    // block ids of the partition (lane b holds block b) and this lane's q chunks
-    const uint32_t my_bt =
-        lane < nb ? block_tables[(int64_t)s * block_table_stride + b_begin + lane] : 0u;
-    constexpr int QV = kF8 ? 2 : 1;  // 16-byte vectors of q per chunk
-    uint4 qv[G][KPL][QV];
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      const T* qrow = query + ((int64_t)s * num_heads + j * G + g) * D;
-#pragma unroll
-      for (int k = 0; k < KPL; ++k)
-#pragma unroll
-        for (int h2 = 0; h2 < QV; ++h2)
-          qv[g][k][h2] =
-              *reinterpret_cast<const uint4*>(qrow + (lane / BS + k * LPT) * X + 8 * h2);
-    }
-
-    // the new K and V rows of head j (the appending wave's lanes 0 .. 2 NR - 1),
-    // loaded before the first tiles so that the wait for those covers them
-    uint4 nrow = make_uint4(0u, 0u, 0u, 0u);
-    if (kAppend && app && lane < 2 * NR)
-      nrow = *reinterpret_cast<const uint4*>(
-          lane < NR ? new_key + (int64_t)s * new_key_stride + (int64_t)j * D + lane * 8
-                    : new_value + (int64_t)s * new_value_stride + (int64_t)j * D +
-                          (lane - NR) * 8);
-
-    // j counts kv_rep replicas of every kv head (more query heads per kv
-    // head than G): its cache head is j / kv_rep
-    const int64_t head_off = (int64_t)(j / kv_rep) * head_stride;
-    const uint4* kbase = reinterpret_cast<const uint4*>(key_cache + head_off);
-    const uint4* vbase = reinterpret_cast<const uint4*>(value_cache + head_off);
-    const int64_t bstride_v = block_stride / X;
-    const int t = lane % BS;     // K: token of this lane within a tile
-    const int seg = lane % VPR;  // V: 8-token segment of this lane
-    const int nks = (((nb + BKS - 1) / BKS) + 1) & ~1;  // stages per pass, rounded up to even
-    float* const my_logit = &s_logit[wave][0][0];
-    uint16_t* const my_p = &s_p[wave][0][0];
-
-    // Block id of tile u of stage st (uniform); blocks past the partition
-    // or out of the pool read block 0 (in bounds) and are masked when
-    // consumed, so loads never branch.
-    // (the pool check compares 32 bits, in scalar registers, unless the
-    // pool holds more than 2^32 blocks)
-    const bool huge_pool = num_blocks > (int64_t)0xffffffffu;
-    auto tile_block = [&](int st, int u, bool& ok) -> uint32_t {
-      const int bi = st * BKS + u;
-      const uint32_t phys = (uint32_t)__builtin_amdgcn_readlane((int)my_bt, bi < nb ? bi : 0);
-      ok = bi < nb && (huge_pool || phys < (uint32_t)num_blocks);
-      return ok ? phys : 0u;
-    };
-    auto load_stage = [&](const uint4* base, int st, uint4(&buf)[NV]) {
-#pragma unroll
-      for (int u = 0; u < BKS; ++u) {
-        bool ok;
-        const uint4* tp = base + (int64_t)tile_block(st, u, ok) * bstride_v + lane;
-#pragma unroll
-        for (int k = 0; k < KPL; ++k) buf[u * KPL + k] = tile_load(tp + 64 * k);
-      }
-    };
-    // logits of BKS tiles
-    auto compute_k = [&](int st, const uint4(&buf)[NV]) {
-#pragma unroll
-      for (int u = 0; u < BKS; ++u) {
-        bool ok;
-        const uint32_t phys = tile_block(st, u, ok);
-        const int bi = st * BKS + u;
-        const bool valid = ok && (b_begin + bi) * BS + t < L;
-        uint4 kt[KPL];
-#pragma unroll
-        for (int k = 0; k < KPL; ++k) kt[k] = buf[u * KPL + k];
-        if constexpr (kAppend) {
-          if (app && ok && bi == nb - 1) {  // (uniform) the new token's block
-            // lane l holds chunk l / BS + k LPT of token t: the token's
-            // lanes take the new row's chunks, then the lanes of its 32-byte
-            // sectors write them back whole
-            if (t == app_off)
-#pragma unroll
-              for (int k = 0; k < KPL; ++k) kt[k] = s_new[lane / BS + k * LPT];
-            if ((t >> 1) == (app_off >> 1)) {
-              uint4* dst = const_cast<uint4*>(kbase) + (int64_t)phys * bstride_v + lane;
-#pragma unroll
-              for (int k = 0; k < KPL; ++k) tile_store(dst + 64 * k, kt[k]);
-            }
-          }
-        }
-        float qk[G];
-#pragma unroll
-        for (int g = 0; g < G; ++g) qk[g] = 0.f;
-#pragma unroll
-        for (int k = 0; k < KPL; ++k) {
-          if constexpr (kF8) {
-            uint4 klo, khi;
-            fp8x16_to_pk<T>(kt[k], klo, khi);
-#pragma unroll
-            for (int g = 0; g < G; ++g)
-              qk[g] = dot16<T>(qv[g][k][1], khi, dot16<T>(qv[g][k][0], klo, qk[g]));
-          } else {
-#pragma unroll
-            for (int g = 0; g < G; ++g) qk[g] = dot16<T>(qv[g][k][0], kt[k], qk[g]);
-          }
-        }
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-          const float r = sum_lanes_mod<BS>(qk[g]);
-          if (lane < BS && bi < PB) my_logit[g * PT + bi * BS + lane] = valid ? r * scale : -INFINITY;
-        }
-      }
-    };
-    // P.V over BKS tiles
-    auto compute_v = [&](int st, const uint4(&buf)[NV]) {
-#pragma unroll
-      for (int u = 0; u < BKS; ++u) {
-        bool ok;
-        const uint32_t phys = tile_block(st, u, ok);
-        if (!ok) continue;
-        const int bi = st * BKS + u;
-        uint4 vv[NVV];
-#pragma unroll
-        for (int k = 0; k < NVV; ++k) vv[k] = buf[u * KPL + k];
-        if constexpr (kAppend) {
-          if (app && bi == nb - 1) {  // (uniform) the new token's block
-            // lane l holds rows l / VPR + k DSTEP, tokens seg X .. seg X + X - 1:
-            // the lanes of the token's segment put in its values, then the
-            // whole tile is written back
-            if (seg == app_off / X) {
-              const uint16_t* nv = reinterpret_cast<const uint16_t*>(&s_new[NR]);
-#pragma unroll
-              for (int k = 0; k < NVV; ++k)
-                vv[k] = put_u16(vv[k], app_off % X, nv[lane / VPR + k * DSTEP]);
-            }
-            uint4* dst = const_cast<uint4*>(vbase) + (int64_t)phys * bstride_v + lane;
-#pragma unroll
-            for (int k = 0; k < NVV; ++k) tile_store(dst + 64 * k, vv[k]);
-          }
-        }
-        if constexpr (kPairRows) {
-          // vector k of lane l: rows 2 (l + 64 k) and 2 (l + 64 k) + 1, the
-          // block's 8 tokens each, against the block's 8 probabilities
-          const int tok0 = (b_begin + bi) * BS;
-#pragma unroll
-          for (int k = 0; k < NVV; ++k) {
-            uint4 vh[2];
-            fp8x16_to_pk<T>(vv[k], vh[0], vh[1]);
-            if (tok0 + BS > L) {  // past the context in the last block: stale values
-#pragma unroll
-              for (int h2 = 0; h2 < 2; ++h2) {
-                union {
-                  uint4 v;
-                  uint16_t e[8];
-                } wv;
-                wv.v = vh[h2];
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                  if (tok0 + e >= L) wv.e[e] = 0;
-                vh[h2] = wv.v;
-              }
-            }
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-              const uint4 pk = *reinterpret_cast<const uint4*>(&my_p[g * PT + bi * BS]);
-              acc[g][2 * k] = dot16<T>(pk, vh[0], acc[g][2 * k]);
-              acc[g][2 * k + 1] = dot16<T>(pk, vh[1], acc[g][2 * k + 1]);
-            }
-          }
-          continue;
-        }
-        const int tok0 = (b_begin + bi) * BS + seg * X;
-        if constexpr (kF8) {
-#pragma unroll
-          for (int k = 0; k < NVV; ++k) {
-            uint4 vh[2];
-            fp8x16_to_pk<T>(vv[k], vh[0], vh[1]);
-            if (tok0 + X > L) {  // past the context in the last block: stale values
-#pragma unroll
-              for (int h2 = 0; h2 < 2; ++h2) {
-                union {
-                  uint4 v;
-                  uint16_t e[8];
-                } wv;
-                wv.v = vh[h2];
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                  if (tok0 + 8 * h2 + e >= L) wv.e[e] = 0;
-                vh[h2] = wv.v;
-              }
-            }
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-              const uint4* pp = reinterpret_cast<const uint4*>(&my_p[g * PT + bi * BS + seg * X]);
-              acc[g][k] = dot16<T>(pp[1], vh[1], dot16<T>(pp[0], vh[0], acc[g][k]));
-            }
-          }
-          continue;
-        }
-        if (tok0 + X > L) {
-          // past the context in the last block: zero the values (stale contents)
-#pragma unroll
-          for (int k = 0; k < NVV; ++k) {
-            union {
-              uint4 v;
-              uint16_t e[8];
-            } wv;
-            wv.v = vv[k];
-#pragma unroll
-            for (int e = 0; e < X; ++e)
-              if (tok0 + e >= L) wv.e[e] = 0;
-            vv[k] = wv.v;
-          }
-        }
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-          const uint4 pk = *reinterpret_cast<const uint4*>(&my_p[g * PT + bi * BS + seg * X]);
-#pragma unroll
-          for (int k = 0; k < NVV; ++k) acc[g][k] = dot16<T>(pk, vv[k], acc[g][k]);
-        }
-      }
-    };
-
-    // ---- software pipeline (nks even): the next stage's loads are in
-    // flight while the current stage is computed; the first two V stages are
-    // issued during the last two K stages, before the softmax ----
-    uint4 bufA[NV], bufB[NV];
-    load_stage(kbase, 0, bufA);
-    load_stage(kbase, 1, bufB);
-    if (kAppend && app) {
-      if (lane < 2 * NR) s_new[lane] = nrow;
-      lds_wave_sync();
-    }
-    for (int st = 0; st + 2 < nks; st += 2) {
-      compute_k(st, bufA);
-      load_stage(kbase, st + 2, bufA);
-      compute_k(st + 1, bufB);
-      load_stage(kbase, st + 3, bufB);
-    }
-    compute_k(nks - 2, bufA);
-    load_stage(vbase, 0, bufA);
-    compute_k(nks - 1, bufB);
-    load_stage(vbase, 1, bufB);
-
-    // ---- softmax over the partition ----
-    lds_wave_sync();
-    {
-      const int ntok = nb * BS;
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        float v[NPL];
-        float mx = -INFINITY;
-#pragma unroll
-        for (int i = 0; i < NPL; ++i) {
-          const int idx = i * 64 + lane;
-          v[i] = idx < ntok ? my_logit[g * PT + idx] : -INFINITY;
-          mx = fmaxf(mx, v[i]);
-        }
-        mx = wave_max_dpp(mx);
-        float sm = 0.f;
-#pragma unroll
-        for (int i = 0; i < NPL; ++i) {
-          if (i * 64 >= ntok) break;  // (uniform) the P.V pass reads only the first ntok
-          const float p = v[i] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(v[i] - mx);
-          sm += p;
-          T pt;
-          store_from_f32<T>(&pt, p);
-          my_p[g * PT + i * 64 + lane] = pt.x;
-        }
-        m[g] = mx;
-        lsum[g] = wave_sum_dpp(sm);
-      }
-    }
-    lds_wave_sync();
-
-    for (int st = 0; st + 2 < nks; st += 2) {
-      compute_v(st, bufA);
-      load_stage(vbase, st + 2, bufA);
-      compute_v(st + 1, bufB);
-      load_stage(vbase, st + 3, bufB);
-    }
-    compute_v(nks - 2, bufA);
-    compute_v(nks - 1, bufB);
-
-    // sum the VPR lanes that hold the same value row
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-      for (int k = 0; k < NACC; ++k) {
-        if constexpr (VPR >= 2) acc[g][k] += dpp<kDppQuadXor1>(acc[g][k]);
-        if constexpr (VPR >= 4) acc[g][k] += dpp<kDppQuadXor2>(acc[g][k]);
-        if constexpr (kF8) acc[g][k] *= vs;
-      }
-  }
-
-  // ---- merge the NW partitions of the chunk in LDS ----
-  // Each wave leaves its unnormalised output (in its own s_logit slot, free
-  // after the softmax) and its max / sum; then the workgroup combines them.
-  // The barriers wait for LDS only: __syncthreads() would also wait for this
-  // wave's outstanding global stores (the fused append's sector writes),
-  // which nothing here reads.
-  lds_barrier();
-  {
-    float* my_row = &s_logit[wave][0][0];
-    if constexpr (kPairRows) {
-#pragma unroll
-      for (int g = 0; g < G; ++g)
-#pragma unroll
-        for (int k = 0; k < NACC; ++k) my_row[g * D + 2 * (lane + 64 * (k / 2)) + k % 2] = acc[g][k];
-    } else {
-      const int row0 = lane / VPR;
-      if (lane % VPR == 0) {
-#pragma unroll
-        for (int g = 0; g < G; ++g)
-#pragma unroll
-          for (int k = 0; k < NVV; ++k) my_row[g * D + row0 + k * DSTEP] = acc[g][k];
-      }
-    }
-    if (lane == 0) {
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        s_m[wave][g] = m[g];
-        s_l[wave][g] = lsum[g];
-      }
-    }
-  }
-  lds_barrier();
-  // thread e of the workgroup combines output elements e, e + 64*NW, ...
-  // (contiguous per head row, so stores write whole lines)
-  const bool single = nchunks == 1;
-  for (int e = threadIdx.x; e < G * D; e += 64 * NW) {
-    const int g = e / D, d = e - (e / D) * D;
-    float mx = -INFINITY;
-#pragma unroll
-    for (int q = 0; q < NW; ++q) mx = fmaxf(mx, s_m[q][g]);
-    float num = 0.f, den = 0.f;
-#pragma unroll
-    for (int q = 0; q < NW; ++q) {
-      const float wq = s_m[q][g] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s_m[q][g] - mx);
-      num = fmaf(wq, s_logit[q][0][g * D + d], num);
-      den = fmaf(wq, s_l[q][g], den);
-    }
-    const int h = j * G + g;
-    if (single) {
-      store_from_f32<T>(out + ((int64_t)s * num_heads + h) * D + d, num / (den + 1e-6f));
-    } else {
-      // split-K partial row: D floats of unnormalised output, then one
-      // 128-byte line {max, sum, 0...} (whole lines: partial-line stores
-      // cost a read-modify-write in HBM)
-      float* prow = part_out + (((int64_t)s * num_heads + h) * max_parts + chunk) * kPartRow<D>;
-      prow[d] = num;
-      if (d < 32) prow[D + d] = d == 0 ? mx : (d == 1 ? den : 0.f);
-    }
-  }
-}
-
 // One wave per (query head, sequence) with more than one partition: merge of
 // the generic kernel's split-K partials.
 template <typename T, int D>
@@ -1164,9 +607,26 @@ constexpr int kF8Waves = VPA_DECODE_FP8_WAVES;
 constexpr int kF8PT = VPA_DECODE_FP8_PT;
 static_assert(kRowsPT >= kDecodeMinPartitionTokens && kF8PT >= kDecodeMinPartitionTokens,
               "workspace sized for 128-token partitions");
-// Tokens per work item (workgroup) of the plan.
+// Largest number of tokens per work item (workgroup) of the list form.
 constexpr int kDecodeChunk = kRowsPT * kRowsWaves;
 static_assert(kF8PT * kF8Waves == kDecodeChunk, "one work list serves every cache type");
+
+// Tokens per work item: half the largest chunk up to 512 (sequence, kv head)
+// pairs, where the longest item is the tail (us per layer, bf16, 2048-token
+// chunks -> 1024; 32 sequences geometric around 800 tokens 30.8 -> 21.5, 64
+// 48.3 -> 44.9; 32 x 3000-4000 77.4 -> 76.5), the largest above (256 x
+// geometric 158.6 -> 165.7) and where it makes the merge launch unnecessary
+// (32 x 100-1500 with appends 26.1 -> 26.7). From host values that
+// the plan, the decode and the read-ceiling calls of a step share
+// (num_kv_heads: replicas included; a workspace laid out for the largest
+// chunk only, max_parts, keeps that).
+int list_chunk(int num_seqs, int num_kv_heads, int max_ctx, int max_parts) {
+  constexpr int kHalf = kDecodeChunk / 2;
+  return max_ctx > kDecodeChunk && (int64_t)num_seqs * num_kv_heads <= 512 &&
+                 max_parts >= (max_ctx + kHalf - 1) / kHalf
+             ? kHalf
+             : kDecodeChunk;
+}
 
 // Merge of split-K partials: persistent waves over (sequence, query head)
 // units; sequences of one chunk were written directly and are skipped. One
@@ -1175,16 +635,25 @@ static_assert(kF8PT * kF8Waves == kDecodeChunk, "one work list serves every cach
 // (the context length, then its partials) before the store.
 constexpr int kMergeRows = 8;
 
+// small_target > 0: partials of the small-grid form, whose chunk length is
+// worked out as its workgroups did (small_chunk_blocks).
 template <typename T, int D>
 __global__ __launch_bounds__(64) void decode_merge_kernel(
     T* __restrict__ out, const uint32_t* __restrict__ context_lens, int32_t num_seqs,
     int32_t max_ctx, int32_t cap_tokens, int32_t part_tokens, int32_t num_heads,
-    const float* __restrict__ part, int32_t max_parts) {
+    const float* __restrict__ part, int32_t max_parts, int32_t small_target,
+    int32_t num_kv_heads, int32_t block_size) {
   constexpr int DPL = (D + 63) / 64;  // output elements per lane (the last partly, at D 96)
   constexpr int RS = kPartRow<D>;
   constexpr int R = kMergeRows;
   const int lane = threadIdx.x;
   const uint32_t units = (uint32_t)num_seqs * (uint32_t)num_heads;
+  if (small_target > 0) {
+    const int L = lane < num_seqs ? clamp_context(context_lens[lane], max_ctx, cap_tokens) : 0;
+    part_tokens = block_size * small_chunk_blocks((max(L, 0) + block_size - 1) / block_size,
+                                                  num_seqs, num_kv_heads, small_target,
+                                                  block_size);
+  }
   for (uint32_t u = blockIdx.x; u < units; u += gridDim.x) {
     const int s = (int)(u / (uint32_t)num_heads);
     const int h = (int)(u % (uint32_t)num_heads);
@@ -1232,10 +701,35 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(
   }
 }
 
-// Shapes whose rows kernel takes the fused append: at least 2 KiB of 16-bit
-// (block, head) tile, i.e. at most two tiles per 8-load stage (more tiles per
-// stage spill scalar registers with the append's extra state).
-constexpr bool fused_append_shape(int d, int bs) { return d * bs >= 2048; }
+// Merge of the partial rows of chunks of part_tokens tokens (or, with
+// small_target, of the small-grid form's).
+template <typename T, int D>
+hipError_t launch_merge_t(void* out, const uint32_t* cl, int32_t num_seqs, int32_t max_ctx,
+                          int32_t cap_tokens, int part_tokens, int32_t num_heads,
+                          const CacheGeom& g, const DecodeWorkspace& ws, int small_target,
+                          hipStream_t stream) {
+  const int64_t units = (int64_t)num_seqs * num_heads;
+  const int64_t waves =
+      std::min<int64_t>(units, (int64_t)device_cu_count() * VPA_DECODE_MERGE_WAVES_PER_CU);
+  hipLaunchKernelGGL((decode_merge_kernel<T, D>), dim3((unsigned)waves), dim3(64), 0, stream,
+                     static_cast<T*>(out), cl, num_seqs, max_ctx, cap_tokens, part_tokens,
+                     num_heads, ws.part_out, ws.max_parts, small_target, g.num_kv_heads,
+                     g.block_size);
+  return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_merge(const DecodeArgs& a, const CacheGeom& g, const DecodeWorkspace& ws,
+                        int small_target, hipStream_t stream) {
+  const int cap = a.block_table_stride * g.block_size;
+#define VPA_MERGE_D(DV)                                                                        \
+  if (g.head_dim == DV)                                                                        \
+    return launch_merge_t<T, DV>(a.out, a.context_lens, a.num_seqs, a.max_ctx, cap, 0,         \
+                                 a.num_heads, g, ws, small_target, stream);
+  VPA_MERGE_D(64) VPA_MERGE_D(96) VPA_MERGE_D(128) VPA_MERGE_D(192) VPA_MERGE_D(256)
+#undef VPA_MERGE_D
+  return hipErrorInvalidValue;
+}
 
 template <typename T, typename C, int D, int BS, int G>
 hipError_t launch_decode_rows_c(void* out, const void* q, const void* kc, const void* vc,
@@ -1247,17 +741,18 @@ hipError_t launch_decode_rows_c(void* out, const void* q, const void* kc, const 
   constexpr bool kFp8 = std::is_same_v<C, fp8_t>;
   constexpr int PT = kFp8 ? kF8PT : kRowsPT;
   constexpr int NW = kFp8 ? kF8Waves : kRowsWaves;
-  constexpr int kChunk = PT * NW;  // tokens per workgroup
-  static_assert(kChunk == kDecodeChunk, "the plan's chunk");
+  static_assert(PT * NW == kDecodeChunk, "the largest chunk");
+  // tokens per workgroup
+  const int chunk = list_chunk(num_seqs, g.num_kv_heads, max_ctx, ws.max_parts);
   const int cap_tokens = bts * g.block_size;
   hipError_t e = hipSuccess;
   if (!ws.planned) {
     hipLaunchKernelGGL(decode_plan_kernel, dim3(1), dim3(1024), 0, stream, cl, num_seqs,
-                       max_ctx, cap_tokens, kChunk, ws.items, ws.queue);
+                       max_ctx, cap_tokens, chunk, ws.items, ws.queue);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  const int max_chunks = max(1, (max_ctx + kChunk - 1) / kChunk);
+  const int max_chunks = max(1, (max_ctx + chunk - 1) / chunk);
   const int64_t units = (int64_t)num_seqs * max_chunks * g.num_kv_heads;
   if constexpr (!kFp8 && fused_append_shape(D, BS)) {
     if (app != nullptr) {
@@ -1269,7 +764,7 @@ hipError_t launch_decode_rows_c(void* out, const void* q, const void* kc, const 
                          ws.max_parts, ws.items, ws.queue, num_seqs, max_ctx, cap_tokens,
                          k_scale, v_scale, static_cast<const T*>(app->key),
                          static_cast<const T*>(app->value), app->key_token_stride,
-                         app->value_token_stride, g.kv_rep);
+                         app->value_token_stride, g.kv_rep, cl, 0, 0);
     }
   }
   if (kFp8 || !fused_append_shape(D, BS) || app == nullptr) {
@@ -1280,17 +775,12 @@ hipError_t launch_decode_rows_c(void* out, const void* q, const void* kc, const 
                        g.num_blocks, g.block_stride, g.head_stride, ws.part_out, ws.max_parts,
                        ws.items, ws.queue, num_seqs, max_ctx, cap_tokens, k_scale, v_scale,
                        static_cast<const T*>(nullptr), static_cast<const T*>(nullptr),
-                       (int64_t)0, (int64_t)0, g.kv_rep);
+                       (int64_t)0, (int64_t)0, g.kv_rep, cl, 0, 0);
   }
   e = hipGetLastError();
   if (e != hipSuccess || max_chunks <= 1) return e;
-  const int64_t munits = (int64_t)num_seqs * num_heads;
-  const int64_t mwaves =
-      std::min<int64_t>(munits, (int64_t)device_cu_count() * VPA_DECODE_MERGE_WAVES_PER_CU);
-  hipLaunchKernelGGL((decode_merge_kernel<T, D>), dim3((unsigned)mwaves), dim3(64), 0, stream,
-                     static_cast<T*>(out), cl, num_seqs, max_ctx, cap_tokens, kChunk, num_heads,
-                     ws.part_out, ws.max_parts);
-  return hipGetLastError();
+  return launch_merge_t<T, D>(out, cl, num_seqs, max_ctx, cap_tokens, chunk, num_heads, g, ws, 0,
+                              stream);
 }
 
 template <typename T, int D, int BS, int G>
@@ -1497,9 +987,9 @@ __global__ __launch_bounds__(64 * kRowsWaves) void paged_read_kernel(
     const uint32_t* __restrict__ block_tables, int32_t block_table_stride,
     int32_t num_kv_heads, int64_t num_blocks, int64_t block_stride_v, int64_t head_stride_v,
     const uint2* __restrict__ items, const uint32_t* __restrict__ queue, int32_t num_seqs,
-    int32_t max_ctx, int32_t cap_tokens, uint32_t magic, uint32_t* __restrict__ sink) {
+    int32_t max_ctx, int32_t cap_tokens, uint32_t magic, uint32_t* __restrict__ sink,
+    int32_t chunk_blocks) {
   constexpr int NW = kRowsWaves;
-  constexpr int PB = kRowsPT / BS;  // blocks per wave partition
   constexpr int NV = VPA_READ_NV;    // loads per lane per stage
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -1516,10 +1006,10 @@ __global__ __launch_bounds__(64 * kRowsWaves) void paged_read_kernel(
   const int L = clamp_context(item.y, max_ctx, cap_tokens);
   if (L <= 0) return;
   const int nblk = (L + BS - 1) / BS;
-  const int nchunks = (nblk + PB * NW - 1) / (PB * NW);
+  const int nchunks = (nblk + chunk_blocks - 1) / chunk_blocks;
   if (chunk >= nchunks) return;
-  const int c_begin = chunk * PB * NW;
-  const int c_nb = min(PB * NW, nblk - c_begin);
+  const int c_begin = chunk * chunk_blocks;
+  const int c_nb = min(chunk_blocks, nblk - c_begin);
   const int b_begin = c_begin + (c_nb * wave) / NW;
   const int nb = c_begin + (c_nb * (wave + 1)) / NW - b_begin;
   if (nb <= 0) return;
@@ -1565,14 +1055,16 @@ hipError_t launch_read_t(const void* kc, const void* vc, const uint32_t* bt, int
                          int32_t max_ctx, int32_t num_seqs, const CacheGeom& g, int elem_bytes,
                          const DecodeWorkspace& ws, uint32_t magic, uint32_t* sink,
                          hipStream_t stream) {
-  const int max_chunks = max(1, (max_ctx + kDecodeChunk - 1) / kDecodeChunk);
+  const int chunk =
+      list_chunk(num_seqs, g.num_kv_heads * g.kv_rep, max_ctx, ws.max_parts);
+  const int max_chunks = max(1, (max_ctx + chunk - 1) / chunk);
   const int64_t units = (int64_t)num_seqs * max_chunks * g.num_kv_heads;
   const int64_t per_vec = 16 / elem_bytes;
   hipLaunchKernelGGL((paged_read_kernel<BS, KPL>), dim3((unsigned)units), dim3(64 * kRowsWaves),
                      0, stream, static_cast<const uint4*>(kc), static_cast<const uint4*>(vc), bt,
                      bts, g.num_kv_heads, g.num_blocks, g.block_stride / per_vec,
                      g.head_stride / per_vec, ws.items, ws.queue, num_seqs, max_ctx,
-                     bts * g.block_size, magic, sink);
+                     bts * g.block_size, magic, sink, chunk / BS);
   return hipGetLastError();
 }
 
@@ -1612,7 +1104,9 @@ hipError_t launch_decode_plan(int dtype, const uint32_t* context_lens, int32_t m
   const bool rows = decode_uses_rows_kernel(dtype, g.head_dim, g.block_size);
   if (!rows || num_seqs == 0) return hipSuccess;
   hipLaunchKernelGGL(decode_plan_kernel, dim3(1), dim3(1024), 0, stream, context_lens, num_seqs,
-                     max_context_len, block_table_stride * g.block_size, kDecodeChunk, ws.items,
+                     max_context_len, block_table_stride * g.block_size,
+                     list_chunk(num_seqs, g.num_kv_heads * g.kv_rep, max_context_len, ws.max_parts),
+                     ws.items,
                      ws.queue);
   return hipGetLastError();
 }
@@ -1741,6 +1235,20 @@ hipError_t launch_paged_decode(int dtype, int cache_dtype, void* out, const void
   CacheGeom gv = g;
   gv.kv_rep = num_heads / g.num_kv_heads / group;
   gv.num_kv_heads = g.num_kv_heads * gv.kv_rep;
+  // (f32 queries, and the tiles above 8 KiB, run the generic kernel)
+  const int target = decode_uses_rows_kernel(dtype, g.head_dim, g.block_size)
+                         ? decode_small_target(num_seqs, gv.num_kv_heads, max_context_len,
+                                               ws.max_parts)
+                         : -1;
+  if (target >= 0) {
+    const DecodeArgs a{out, query, key_cache, value_cache, block_tables, block_table_stride,
+                       context_lens, max_context_len, scale, num_seqs, num_heads, k_scale,
+                       v_scale, append};
+    const hipError_t e = launch_decode_small(dtype, cache_dtype, group, a, gv, ws, target, stream);
+    if (e != hipSuccess || target == 0) return e;
+    return dtype == VPA_DTYPE_BF16 ? launch_merge<bf16_t>(a, gv, ws, target, stream)
+                                   : launch_merge<f16_t>(a, gv, ws, target, stream);
+  }
   if (cache_dtype == VPA_DTYPE_FP8_E4M3)
     return dispatch_decode_fp8(dtype, g.head_dim, g.block_size, group, out, query, key_cache,
                                value_cache, block_tables, block_table_stride, context_lens,

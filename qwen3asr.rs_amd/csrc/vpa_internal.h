@@ -43,7 +43,7 @@ struct DecodeWorkspace {
   float* part_max;   // [num_seqs, num_heads, max_parts]
   float* part_sum;   // [num_seqs, num_heads, max_parts]
   uint2* items;      // [num_seqs * max(1, max_parts)] work list {seq << 16 | partition, length}
-  uint32_t* queue;   // [2]: next work unit, number of items
+  uint32_t* queue;   // [2]: log2 of the list's chunk in tokens, number of items
   int max_parts;     // ceil(max_context_len / partition tokens of the layout)
   bool planned = false;  // the work list is already in the workspace (skip the plan launch)
 };
@@ -70,6 +70,13 @@ bool decode_fuses_append(int dtype, int cache_dtype, int head_dim, int block_siz
 // Query heads per kv head a decode kernel instance serves for G query heads
 // per kv head (4, 2 or 1, dividing G); larger G runs G / that replicas.
 int decode_kernel_group(int group);
+// Replicas of each kv head that decode with that many query heads per group
+// (at least 1).
+inline int decode_kv_rep(int num_heads, int num_kv_heads) {
+  const int group = num_heads / num_kv_heads;
+  const int rep = group / decode_kernel_group(group);
+  return rep > 0 ? rep : 1;
+}
 
 // Compute units of the current device (cached per device).
 int device_cu_count();
@@ -162,6 +169,33 @@ hipError_t launch_gather_kv_cache(int cache_dtype, int out_dtype, void* out_key,
                                   int32_t block_table_stride, const uint32_t* cu_seqlens,
                                   int32_t num_seqs, const CacheGeom& g, const float* k_scale,
                                   const float* v_scale, hipStream_t stream);
+
+// Arguments of one decode, for the launchers behind launch_paged_decode.
+struct DecodeArgs {
+  void* out;
+  const void* query;
+  const void* key_cache;
+  const void* value_cache;
+  const uint32_t* block_tables;
+  int32_t block_table_stride;
+  const uint32_t* context_lens;
+  int32_t max_ctx;
+  float scale;
+  int32_t num_seqs;
+  int32_t num_heads;
+  const float* k_scale;
+  const float* v_scale;
+  const DecodeAppend* append;
+};
+// The rows kernel's form for small grids (decode_small_kernels.hip): whether
+// a call takes it (-1: no; 0: every context in one chunk, no merge launch;
+// else the number of workgroups its chunk length aims at), from the host's
+// values alone (num_kv_heads: replicas included), and its launch.
+constexpr int kSmallMaxSeqs = 64;
+int decode_small_target(int num_seqs, int num_kv_heads, int max_ctx, int max_parts);
+hipError_t launch_decode_small(int dtype, int cache_dtype, int group, const DecodeArgs& a,
+                               const CacheGeom& g, const DecodeWorkspace& ws, int target,
+                               hipStream_t stream);
 
 // cache_dtype is dtype, or VPA_DTYPE_FP8_E4M3 with a bf16 / f16 query
 // (scales are device pointers, read only for fp8).
