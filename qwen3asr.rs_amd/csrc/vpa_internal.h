@@ -218,6 +218,30 @@ hipError_t launch_prefill_paged(int dtype, int cache_dtype, void* out, const voi
                                 const float* k_scale, const float* v_scale,
                                 hipStream_t stream);
 
+// Arguments of the 16-bit MFMA prefill after its checks.
+struct PrefillArgs {
+  void* out;
+  const void* query;
+  const void* key_cache;
+  const void* value_cache;
+  const uint32_t* block_tables;
+  int32_t block_table_stride;
+  const uint32_t* cu_seqlens_q;
+  const uint32_t* context_lens;
+  int32_t num_seqs, max_query_len, max_kv_len;
+  int64_t total_query_rows;
+  float scale;
+  float denom_eps;
+  int32_t causal, num_heads;
+  const float* k_scale;
+  const float* v_scale;
+};
+// The form for few rows (prefill_split_kernels.hip): whether a call takes it,
+// and its launch.
+bool prefill_split_keys(const PrefillArgs& a, const CacheGeom& g);
+hipError_t launch_prefill_split(int dtype, int cache_dtype, const PrefillArgs& a,
+                                const CacheGeom& g, hipStream_t stream);
+
 // The f32 prefill on the f32 matrix instructions (prefill_f32_kernels.hip):
 // f32 queries over f32 or fp8 caches, every shape. Same arguments.
 hipError_t launch_prefill_f32(int dtype, int cache_dtype, void* out, const void* query,
