@@ -49,7 +49,9 @@ def _err(msg: str):
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    # the raw handle of torch.cuda.current_stream(t.device), without building
+    # the Stream object around it on every call
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -57,16 +59,16 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 
 def _require_device(*ts: torch.Tensor) -> None:
-    dev = None
+    first = None
     for t in ts:
         if t is None:
             continue
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise _err(f"tensor on {t.device}: paged-KV ops run on the GPU only")
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise _err(f"device mismatch: {dev} vs {t.device}")
+        if first is None:
+            first, dev = t, t.get_device()
+        elif t.get_device() != dev:
+            raise _err(f"device mismatch: {first.device} vs {t.device}")
 
 
 def cache_geometry(key_cache: torch.Tensor, value_cache: torch.Tensor):
@@ -179,10 +181,11 @@ def paged_attention(q: torch.Tensor, k_scale: Optional[torch.Tensor],
     elif out.shape != q.shape or out.dtype != q.dtype or not out.is_contiguous():
         raise _err("out must be a contiguous tensor shaped and typed like q")
     lib = _lib.load()
-    need = lib.vpa_paged_attention_workspace_size(b, h, d, int(max_context_len))
-    if workspace is None and need > 0:
-        workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
-    ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
+    if workspace is None:
+        need = lib.vpa_paged_attention_workspace_size(b, h, d, int(max_context_len))
+        if need > 0:
+            workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
+    ws_bytes = 0 if workspace is None else workspace.nbytes
     if planned and workspace is None:
         raise _err("planned=True needs the workspace paged_attention_plan filled")
     fn = lib.vpa_paged_attention_planned if planned else lib.vpa_paged_attention
@@ -238,10 +241,11 @@ def reshape_and_cache_paged_attention(q: torch.Tensor, key: torch.Tensor, value:
     elif out.shape != q.shape or out.dtype != q.dtype or not out.is_contiguous():
         raise _err("out must be a contiguous tensor shaped and typed like q")
     lib = _lib.load()
-    need = lib.vpa_paged_attention_workspace_size(b, h, d, int(max_context_len))
-    if workspace is None and need > 0:
-        workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
-    ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
+    if workspace is None:
+        need = lib.vpa_paged_attention_workspace_size(b, h, d, int(max_context_len))
+        if need > 0:
+            workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
+    ws_bytes = 0 if workspace is None else workspace.nbytes
     if planned and workspace is None:
         raise _err("planned=True needs the workspace paged_attention_plan filled")
     fn = (lib.vpa_reshape_and_cache_paged_attention_planned if planned
