@@ -693,13 +693,17 @@ def traffic_from_profile(w):
 
     path = os.path.join("profiles", f"paged_decode_{w.name}_traffic.json")
     full = os.path.join(ROOT, path)
-    src = os.path.join(ROOT, "qwen3asr.rs_amd", "csrc", "decode_kernels.hip")
+    srcs = [os.path.join(ROOT, "qwen3asr.rs_amd", "csrc", f)
+            for f in ("decode_rows.h", "decode_kernels.hip")]
     if not os.path.exists(full):
         return None, {"source": path, "status": "absent"}
     with open(full) as f:
         j = json.load(f)
-    with open(src, "rb") as f:
-        sha = hashlib.sha256(f.read()).hexdigest()[:16]
+    digest = hashlib.sha256()
+    for src in srcs:
+        with open(src, "rb") as f:
+            digest.update(f.read())
+    sha = digest.hexdigest()[:16]
     measured = j.get("decode_kernels_sha256_16")
     stale = measured != sha
     info = {"source": path, "measured_on_decode_kernels_sha256_16": measured,
