@@ -51,6 +51,8 @@ def _err(msg: str):
 def _stream(t: torch.Tensor) -> int:
     # the raw handle of torch.cuda.current_stream(t.device), without building
     # the Stream object around it on every call
+    if not t.is_cuda:
+        return torch.cuda.current_stream(t.device).cuda_stream  # raises: not a GPU
     return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 

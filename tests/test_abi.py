@@ -515,3 +515,19 @@ def test_fused_append_decode_planned_validates_alike():
         assert rc_a == rc_b != 0
         assert msg_b.replace("_planned", "") == msg_a
     assert fused_call(b=0)[0] == 0
+
+
+def test_state_objects_on_the_cpu_are_refused():
+    """The device-state calls take no tensor argument to check: on host memory
+    they raise before any launch, as torch's current_stream does."""
+    import torch
+
+    import vpa
+
+    state = vpa.DecodeTokenState(2, 4, [1], "cpu")
+    with pytest.raises((ValueError, RuntimeError, AssertionError)):
+        state.consume()
+    alloc = vpa.DeviceBlockAllocator(8, 16, 2, 4, "cpu")
+    with pytest.raises((ValueError, RuntimeError, AssertionError)):
+        alloc.step()
+    assert not torch.any(state.input_ids.view(torch.int32))

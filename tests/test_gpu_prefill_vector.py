@@ -188,7 +188,8 @@ def test_prefill_any_group_infinite_values_and_zero_scale(device, code):
 
 
 @pytest.mark.parametrize("fp8", [False, True])
-@pytest.mark.parametrize("d,bs,n,prior", [(128, 16, 31, 70), (64, 32, 33, 5), (96, 8, 64, 129)])
+@pytest.mark.parametrize("d,bs,n,prior", [(128, 16, 31, 70), (64, 32, 33, 5), (96, 8, 64, 129),
+                                          (192, 32, 20, 40), (256, 16, 34, 30)])
 def test_prefill_f32_many_short_rows(device, d, bs, n, prior, fp8):
     """Many row tiles over at most 320 keys: a wave of the f32 kernel takes a
     row tile of its own instead of a quarter of one tile's keys (the other
