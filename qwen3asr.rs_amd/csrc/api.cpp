@@ -380,8 +380,8 @@ int paged_attention_impl(void* out, const void* query, const float* k_scale,
   ws.planned = planned;
   // The append runs inside the decode launch (the rows kernel's fused form,
   // 16-bit caches) for small batches only: measured on c3's length rule over
-  // 28 layers (us per step, two launches against one), batch 1: 226 / 152,
-  // 8: 651 / 571, 32: 953 / 889, 64: 1425-1459 / 1459, 128: 2437 / 2524,
+  // 28 layers (us per step, two launches against one), batch 1: 214 / 142,
+  // 8: 363 / 284, 32: 741 / 672, and, with 2048-token chunks, 64: 1425-1459 / 1459, 128: 2437 / 2524,
   // 256: 4484 / 4721. Inside a bandwidth-bound decode the token's sector
   // writes interleave with the tile reads and cost more than the append's
   // own launch; with few sequences that launch is what costs. Larger batches
