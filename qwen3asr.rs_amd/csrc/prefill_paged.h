@@ -465,8 +465,11 @@ __attribute__((amdgpu_waves_per_eu(prefill_waves_per_eu<D>()))) void prefill_pag
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
     for (int e = 0; e < 16; ++e) o[dt][e] = 0.f;
-  // (never 0: a masked score is -inf, and 0 * -inf would be NaN)
-  const float sl = fmaxf(fabsf(scale_log2), 1.17549435e-38f);
+  // (never 0: a masked score is -inf, and 0 * -inf would be NaN; by a
+  // comparison, which is false for a NaN scale and keeps it, where fmaxf
+  // would drop it and leave the plain mean of the values)
+  const float abs_scale = fabsf(scale_log2);
+  const float sl = abs_scale < 1.17549435e-38f ? 1.17549435e-38f : abs_scale;
   float m = -INFINITY;   // reference max of the row (moves lazily), log2 units
   float mt = -INFINITY;  // the row's true max so far, log2 units
   float lsum = 0.f;      // this lane's share of the row's exp sum
