@@ -128,40 +128,34 @@ __device__ __forceinline__ void dma16(const void* src, const void* lds) {
 template <int N>
 using Int = std::integral_constant<int, N>;
 
-// Two probabilities as two pairs of T each, high + low parts: high is p
-// rounded toward zero, so the low part is never negative, and it is kept
-// above zero wherever p is (well above T's smallest value): an infinite value
-// then adds +inf times a positive number twice, and the sum stays infinite
-// as it is with the f32 probability. f16 probabilities are scaled by
-// 2^kProbScaleLog2 (and with them the row sums), which moves f16's smallest
-// value to 2^-31 of a probability of 1; bf16 has f32's range.
+// The probabilities of a pair go through the P.V MFMAs as kProbParts pairs of
+// T whose sum they are, taken one after the other: take_part returns the
+// pair's next part and leaves what remains. In bf16 three parts hold the 24
+// bits of an f32 exactly; in f16 two hold 22. Parts are rounded toward zero
+// (f16's last one to nearest), so none is negative, and what remains is kept
+// above zero wherever the probability is: an infinite value then adds +inf
+// times a positive number with each part, and the sum stays infinite as it is
+// with the f32 probability. f16 probabilities are scaled by 2^kProbScaleLog2
+// (and with them the row sums), which moves f16's smallest value to 2^-31 of
+// a probability of 1; bf16 has f32's range.
+template <typename T>
+constexpr int kProbParts = std::is_same_v<T, bf16_t> ? 3 : 2;
 template <typename T>
 constexpr int kProbScaleLog2 = std::is_same_v<T, f16_t> ? 7 : 0;
 
-template <typename T>
-__device__ __forceinline__ uint32_t prob_high(float p0, float p1);
-template <>
-__device__ __forceinline__ uint32_t prob_high<bf16_t>(float p0, float p1) {
-  return (__float_as_uint(p1) & 0xffff0000u) | (__float_as_uint(p0) >> 16);
-}
-template <>
-__device__ __forceinline__ uint32_t prob_high<f16_t>(float p0, float p1) {
-  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(p0, p1));
-}
-template <typename T>
-__device__ __forceinline__ uint32_t prob_low(float p0, float p1, uint32_t high);
-template <>
-__device__ __forceinline__ uint32_t prob_low<bf16_t>(float p0, float p1, uint32_t high) {
-  // (the last bit set: the rest is at least 2^-24 of p)
-  return pack2_hw<bf16_t>(
-      __uint_as_float(__float_as_uint(p0) | 1u) - low_half_f32<bf16_t>(high),
-      __uint_as_float(__float_as_uint(p1) | 1u) - high_half_f32<bf16_t>(high));
-}
-template <>
-__device__ __forceinline__ uint32_t prob_low<f16_t>(float p0, float p1, uint32_t high) {
-  constexpr float kTiny = 5.9604645e-8f;  // 2^-24, f16's smallest value
-  return pack2_hw<f16_t>(fmaxf(p0 - low_half_f32<f16_t>(high), fminf(p0, kTiny)),
-                         fmaxf(p1 - high_half_f32<f16_t>(high), fminf(p1, kTiny)));
+template <typename T, bool kLast>
+__device__ __forceinline__ uint32_t take_part(float& p0, float& p1) {
+  if constexpr (kLast && std::is_same_v<T, f16_t>) return pack2_hw<T>(p0, p1);
+  constexpr bool kBf16 = std::is_same_v<T, bf16_t>;
+  constexpr float kTiny = kBf16 ? 1.17549435e-38f : 5.9604645e-8f;  // T's (normal) smallest
+  uint32_t part;
+  if constexpr (kBf16)
+    part = (__float_as_uint(p1) & 0xffff0000u) | (__float_as_uint(p0) >> 16);
+  else
+    part = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(p0, p1));
+  p0 = fmaxf(p0 - low_half_f32<T>(part), fminf(p0, kTiny));
+  p1 = fmaxf(p1 - high_half_f32<T>(part), fminf(p1, kTiny));
+  return part;
 }
 
 typedef int v4i_t __attribute__((ext_vector_type(4)));
@@ -297,13 +291,19 @@ constexpr int prefill_waves_per_eu() {
 // G: query heads per kv head (1, 2 or 4), or 0: any number of them, given at
 // run time (`group`). G = 0 enumerates the (position, head) rows of a kv head
 // heads-fastest, so a group that does not divide 32 still fills every row of
-// a wave, and keeps 16 (bf16) or 22 (f16) bits of each probability: P goes
-// through the P.V MFMAs as two values of T (prob_high, prob_low), half as
-// many MFMAs again, where the vector kernel kept P in f32. MFMA-bound like
-// the fixed groups. Measured with the append before it (f16, 32 query over
-// 4 kv heads, 12 sequences of 33-450 new over 0-700 prior tokens, 21.2
-// GFLOP): 58.7 us, against 766 us on the vector kernel; error against 64
-// bits 2.1e-4 both ways, the output's rounding.
+// a wave, and keeps the probabilities' f32 bits (f16: 22 of them), as the
+// vector kernel these groups ran on did: P goes through the P.V MFMAs as three
+// values of bf16 or two of f16 (take_part). MFMA-bound like the fixed groups.
+// Measured with the append before it (32 query over 4 kv heads, 12 sequences
+// of 33-450 new over 0-700 prior tokens, 21.2 GFLOP): f16 58.7 us, against 766
+// us on the vector kernel; error against 64 bits 2.07e-4 both ways, the
+// output's rounding. The attention alone of 12 sequences of 240 new over 350
+// prior tokens: f16 56.4 us (vector kernel 817), bf16 63.1 (949).
+// Why three parts in bf16: with two, 16 bits, the same 12 sequences of 240
+// took 55.0 us, but were 1.658228e-3 off 64 bits with 0.43 % of the outputs
+// not the nearest bf16, where the vector kernel and three parts are
+// 1.658221e-3 off with 0.02 %. A third part in f16 gains nothing (0.216 and
+// 0.217 % not the nearest at 3500 keys) and takes a sixth more time.
 //
 // kSplit: the four waves of a workgroup share one tile of 32 rows and split
 // its keys, tile 4 t + w to wave w, each with its own online softmax, merged
@@ -688,21 +688,25 @@ __attribute__((amdgpu_waves_per_eu(prefill_waves_per_eu<D>()))) void prefill_pag
 #pragma unroll
     for (int r = 1; r < 16; ++r) ps += sval[r];
     lsum += ps;
+    // (n: part of the probabilities, kAnyGroup; taken one at a time, so that
+    // one part's operands are live)
     uint4 pk[2];
-    uint4 pl[kAnyGroup ? 2 : 1];  // kAnyGroup: what pk left of the probabilities
+    auto pack = [&](auto n) {
 #pragma unroll
-    for (int k2 = 0; k2 < 2; ++k2) {
-      const float* p = sval + 8 * k2;
-      if constexpr (kAnyGroup) {
-        pk[k2] = make_uint4(prob_high<T>(p[0], p[1]), prob_high<T>(p[2], p[3]),
-                            prob_high<T>(p[4], p[5]), prob_high<T>(p[6], p[7]));
-        pl[k2] = make_uint4(prob_low<T>(p[0], p[1], pk[k2].x), prob_low<T>(p[2], p[3], pk[k2].y),
-                            prob_low<T>(p[4], p[5], pk[k2].z), prob_low<T>(p[6], p[7], pk[k2].w));
-      } else {
-        pk[k2] = make_uint4(pack2_hw<T>(p[0], p[1]), pack2_hw<T>(p[2], p[3]),
-                            pack2_hw<T>(p[4], p[5]), pack2_hw<T>(p[6], p[7]));
+      for (int k2 = 0; k2 < 2; ++k2) {
+        uint32_t w[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float &p0 = sval[8 * k2 + 2 * i], &p1 = sval[8 * k2 + 2 * i + 1];
+          if constexpr (kAnyGroup)
+            w[i] = take_part<T, decltype(n)::value + 1 == kProbParts<T>>(p0, p1);
+          else
+            w[i] = pack2_hw<T>(p0, p1);
+        }
+        pk[k2] = make_uint4(w[0], w[1], w[2], w[3]);
       }
-    }
+    };
+    pack(Int<0>{});
     // k-step k2 of lane half h covers keys 16 k2 + 8h .. 16 k2 + 8h + 7, one
     // unit of row d = 32 dt + col (values of absent keys were zeroed in LDS
     // by the step)
@@ -721,17 +725,21 @@ __attribute__((amdgpu_waves_per_eu(prefill_waves_per_eu<D>()))) void prefill_pag
                                        std::make_integer_sequence<int, DT>{});
       lgkm_wait(vop);
     }
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int k2 = 0; k2 < 2; ++k2)
-        o[dt] = mfma32x32x16<T>(__builtin_bit_cast(uint4, vop[dt][k2]), pk[k2], o[dt]);
-    if constexpr (kAnyGroup) {
+    auto pv = [&] {
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int k2 = 0; k2 < 2; ++k2)
-          o[dt] = mfma32x32x16<T>(__builtin_bit_cast(uint4, vop[dt][k2]), pl[k2], o[dt]);
+          o[dt] = mfma32x32x16<T>(__builtin_bit_cast(uint4, vop[dt][k2]), pk[k2], o[dt]);
+    };
+    pv();
+    if constexpr (kAnyGroup) {
+      pack(Int<1>{});
+      pv();
+      if constexpr (kProbParts<T> == 3) {
+        pack(Int<2>{});
+        pv();
+      }
     }
   };
 

@@ -146,19 +146,53 @@ def test_prefill_any_group_keeps_f32_probabilities(device, code, group, kvh, d, 
     """16-bit queries with any number of query heads per kv head on the MFMA
     kernel: (position, head) row tiles of 128 rows that end inside a position
     (groups that divide neither 32 nor 128, and one above 128), 1 to 129 new
-    tokens. The probabilities keep more than 16 bits: next to the output's
-    own rounding (half a unit in the last place, at most 2^-8 of the value in
-    bf16 and 2^-11 in f16) an element may be off by what the probabilities'
-    two parts leave (2^-17 in bf16, whose parts hold 16 bits; 2^-20 covers
-    f16's 22 bits and the f32 sums) times the largest |value| behind it
-    (below 12 here: 6 standard deviations times the fp8 data's 2)."""
+    tokens. The probabilities keep their f32 bits: next to the output's own
+    rounding (half a unit in the last place, at most 2^-8 of the value in bf16
+    and 2^-11 in f16) an element may be off by 2^-20, which covers f16's 22
+    bits and the f32 sums, times the largest |value| behind it (below 12 here:
+    6 standard deviations times the fp8 data's 2)."""
     got, want = vector_case(device, code, group * kvh, kvh, d, bs, [0, 37, 300, 1], [1, 43, 129, 2],
                             seed=group + d, causal=True, fp8=fp8)
-    half, low = (2.0 ** -8, 2.0 ** -17) if code == orc.BF16 else (2.0 ** -11, 2.0 ** -20)
+    half = 2.0 ** -8 if code == orc.BF16 else 2.0 ** -11
     err = np.abs(got.astype(np.float64) - want)
-    bound = half * np.abs(want) + 12 * low
+    bound = half * np.abs(want) + 12 * 2.0 ** -20
     assert np.all(np.isfinite(got))
     assert np.max(err / bound) <= 1.0, f"worst {np.max(err / bound):.2f} of the bound"
+
+
+@pytest.mark.parametrize("code", [orc.BF16, orc.F16])
+@pytest.mark.parametrize("group,kvh,d,bs", [(3, 2, 128, 16), (8, 1, 64, 32), (5, 2, 256, 16)])
+@pytest.mark.parametrize("n", [40, 600])
+def test_prefill_any_group_cancelling_values(device, code, group, kvh, d, bs, n):
+    """Values of +1 and -1 under nearly equal probabilities: the output is
+    their difference, about 2^-13 of a probability, and shows every bit they
+    are held in. Next to the output's own rounding an element may be off by
+    2^-21: the exponent's rounding (at most 2^-22 of it at f16's offset of 7,
+    times ln 2), the exponential's unit in the last place, f16's two parts
+    (2^-23) and the f32 sums."""
+    h, nq = group * kvh, 9
+    nb = n // bs + 3
+    rng = np.random.default_rng(n + d)
+    kc = np.zeros((nb, kvh, d // 8, bs, 8), np.float32)
+    vc = np.zeros((nb, kvh, d, bs), np.float32)
+    bt = block_tables_for(rng, [n], nb, bs)
+    pos = np.arange(n)
+    blk, off = bt[0, pos // bs], pos % bs
+    plus = (pos % 2 == 0).astype(np.float32)
+    kc[blk, :, 0, off, 0] = (plus * 2.0 ** -12)[:, None]
+    vc[blk, :, :, off] = (2 * plus - 1)[:, None, None]
+    q = np.zeros((nq, h, d), np.float32)
+    q[:, :, 0] = 1 + rng.integers(0, 64, (nq, h)) / 64  # exact in both types
+    kc, vc, qw = (orc.from_f32(x, code) for x in (kc, vc, q))
+    out = vpa.paged_attention_varlen_prefill(
+        to_dev(qw, code, device), to_dev(kc, code, device), to_dev(vc, code, device),
+        u32(bt, device), u32([n], device), u32([0, nq], device), None, None, 1.0, 1.0,
+        causal=False, denom_eps=0.0)
+    got = orc.to_f32(to_host(out), code).astype(np.float64)
+    want = np.broadcast_to(np.tanh(q[:, :, :1].astype(np.float64) * 2.0 ** -13), got.shape)
+    half = 2.0 ** -8 if code == orc.BF16 else 2.0 ** -11
+    err = np.abs(got - want) / (half * np.abs(want) + 2.0 ** -21)
+    assert np.max(err) <= 1.0, f"worst {np.max(err):.2f} of the bound"
 
 
 @pytest.mark.parametrize("code", [orc.BF16, orc.F16])
