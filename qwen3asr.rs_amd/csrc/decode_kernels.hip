@@ -815,12 +815,15 @@ hipError_t launch_decode_tc(void* out, const void* q, const void* kc, const void
                             const float* v_scale, const DecodeAppend*) {
   // Half partitions where whole ones leave most SIMDs without a wave: a wave
   // runs its partition's K and V passes alone, so a small call lasts as long
-  // as one partition (one f32 sequence of 512 tokens over 8 kv heads:
-  // 21.8 -> 17.8 us for the eager call). (A workspace laid out for whole partitions keeps
-  // them.)
+  // as one partition (one f32 sequence of 512 tokens over 8 kv heads: 21.8 ->
+  // 17.8 us for the eager call). Not where one whole partition reaches the
+  // maximum and no merge launch follows it (us per layer, whole -> half; 1 x
+  // 90-129 tokens 10.5 -> 11.9, 1 x 140-200 14.3 -> 14.9, 2 x 26-77 of 256
+  // 7.8 -> 9.3; what this gives up is 1 x 180-256 16.9 -> 14.5). (A workspace
+  // laid out for whole partitions keeps them.)
   constexpr int kHalf = kPT / 2;
   const int64_t whole = (int64_t)num_seqs * g.num_kv_heads * ((max_ctx + kPT - 1) / kPT);
-  const int pt = whole < 2 * (int64_t)device_cu_count() &&
+  const int pt = max_ctx > kPT && whole < 2 * (int64_t)device_cu_count() &&
                          ws.max_parts >= (max_ctx + kHalf - 1) / kHalf
                      ? kHalf
                      : kPT;

@@ -95,3 +95,29 @@ def test_decode_small_grid_append(device, name, h, kvh, d, bs):
     torch.cuda.synchronize()
     for x, y in zip([two] + a, [one] + b):
         assert torch.equal(x.view(torch.int16), y.view(torch.int16))
+
+
+@pytest.mark.parametrize("b,max_ctx,parts", [(1, 1, 0), (1, 129, 0), (3, 200, 0), (2, 256, 0),
+                                             (2, 257, 3), (1, 512, 4), (40, 512, 2)])
+def test_f32_partitions(device, b, max_ctx, parts):
+    """f32 decode: up to one whole partition (256 tokens) a call writes its
+    output alone (no partial rows, so no second launch to merge them); above,
+    half partitions where whole ones leave SIMDs idle, whole ones else.
+    parts: the partial rows of a sequence and head."""
+    h, kvh, d, bs = 16, 8, 64, 16
+    lens = [max_ctx] * b
+    q, kc, vc, bt, lens = setup(device, orc.F32, h, kvh, d, bs, lens, max_ctx, seed=b + max_ctx,
+                                absent=False)
+    ws = vpa.paged_attention_workspace(b, h, d, max_ctx, device)
+    ws.fill_(0xff)
+    out = vpa.paged_attention(
+        to_dev(q, orc.F32, device), None, None, to_dev(kc, orc.F32, device),
+        to_dev(vc, orc.F32, device), u32(bt, device), u32(lens, device), None, max_ctx, d ** -0.5,
+        1.0, None, workspace=ws)
+    torch.cuda.synchronize()
+    want = orc.paged_attention(q, kc, vc, bt, lens, max_ctx, d ** -0.5, dtype=orc.F32)
+    assert_attention_close(to_host(out), want, orc.F32, f"f32 {b} x {max_ctx}")
+    written = int((ws.view(torch.int32) != -1).sum())
+    assert (written > 0) == (parts > 0)
+    # each partial row is head_dim outputs, a maximum and a sum
+    assert abs(written - b * h * parts * (d + 2)) <= written // 100
