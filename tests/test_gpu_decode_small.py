@@ -2,10 +2,12 @@
 list, chunk length worked out on the device) and of the work list's two chunk
 lengths, against the fp64 oracle, at the sizes where each takes over: one
 chunk up to a maximum of 512 tokens; chunks of 256, 512 and 1024 tokens up to
-128 (sequence, kv head) pairs; above, the list, with 1024-token chunks up to
-512 pairs where the maximum exceeds 2048 and 2048-token ones otherwise. Lengths sit on both sides of tiles and
-chunks, with empty contexts, absent blocks and a maximum (as frozen in a
-captured graph) above every length."""
+128 (sequence, kv head) pairs; above, the list, with 2048-token chunks, or
+1024-token ones where the maximum exceeds 2048, there are at most 512 pairs
+and the lengths ask for it. Lengths sit on both sides of tiles and chunks,
+with empty contexts, absent blocks and a maximum (as frozen in a captured
+graph) above every length. The list's cases have enough sequences for it at
+every number of kv heads here."""
 
 import numpy as np
 import pytest
@@ -27,9 +29,10 @@ CASES = {
     "chunk_256_two": ([3000, 2049], 3000),
     "chunk_512": ([1500, 1024, 1537, 1, 0, 1536, 1025, 1999], 2048),
     "chunk_1024": ([3000 + 7 * i for i in range(14)] + [1024, 1025], 4096),
-    "list_1024": ([600 + 91 * i for i in range(16)] + [1024, 2048, 0], 2200),
-    "list_1024_short": ([130 + 5 * i for i in range(40)], 1024),
+    "list_1024": ([600 + 91 * i for i in range(16)] + [1024, 2048, 0] + [90] * 21, 2200),
+    "list_one_chunk": ([130 + 5 * i for i in range(40)], 1024),
     "list_2048": ([(53 * i) % 700 for i in range(64)] + [2048, 2049], 2049),
+    "list_2048_choice": ([1100 + 37 * i for i in range(24)] + [1024, 1] + [300] * 8, 4096),
 }
 
 
@@ -49,7 +52,7 @@ def setup(device, code, h, kvh, d, bs, lens, max_ctx, seed, absent=True):
 
 @pytest.mark.parametrize("name", CASES)
 @pytest.mark.parametrize("code,h,kvh,d,bs", [(orc.BF16, 16, 8, 128, 16), (orc.F16, 16, 4, 64, 32),
-                                             (orc.BF16, 8, 8, 192, 8)])
+                                             (orc.BF16, 8, 8, 192, 8), (orc.BF16, 16, 8, 128, 32)])
 def test_decode_small_grid_and_list(device, name, code, h, kvh, d, bs):
     lens, max_ctx = CASES[name]
     q, kc, vc, bt, lens = setup(device, code, h, kvh, d, bs, lens, max_ctx, seed=len(lens) + d)
@@ -95,6 +98,50 @@ def test_decode_small_grid_append(device, name, h, kvh, d, bs):
     torch.cuda.synchronize()
     for x, y in zip([two] + a, [one] + b):
         assert torch.equal(x.view(torch.int16), y.view(torch.int16))
+
+
+@pytest.mark.parametrize("seqs,kvh,lo,hi,max_ctx", [
+    (40, 8, 1, 700, 4096),     # 1024-token items no more than the CUs
+    (24, 8, 1228, 2048, 4096),  # twice as many items of 1024 as of 2048, which fit the CUs
+    (17, 8, 200, 4096, 4096),
+    (60, 8, 1000, 4096, 4096),  # more items than CUs either way, some beyond 2048
+    (64, 8, 400, 1228, 8192),  # none beyond 2048
+    (24, 8, 1228, 2048, 2048),  # no choice: one chunk reaches the maximum
+    (65, 8, 1, 4096, 4096),    # no choice: more than 512 pairs
+    (200, 1, 900, 3000, 3000)])
+def test_list_chunk_length_follows_the_items(device, seqs, kvh, lo, hi, max_ctx):
+    """The list's header: log2 of its chunk length and the number of items,
+    against the rule worked out here (1024-token chunks where they are no
+    more items than compute units, or where some context exceeds 2048 tokens
+    and 2048-token chunks are more than 9/8 of the units; else 2048), and the
+    decode over it against the oracle."""
+    h, d, bs = 2 * kvh, 64, 16
+    rng = np.random.default_rng(seqs + hi)
+    lens = rng.integers(lo, hi, size=seqs, endpoint=True)
+    lens[:2] = lo, hi
+    q, kc, vc, bt, lens = setup(device, orc.BF16, h, kvh, d, bs, [int(x) for x in lens], max_ctx,
+                                seed=seqs)
+    args = (to_dev(q, orc.BF16, device), None, None, to_dev(kc, orc.BF16, device),
+            to_dev(vc, orc.BF16, device), u32(bt, device), u32(lens, device), None, max_ctx,
+            d ** -0.5, 1.0, None)
+    ws = vpa.paged_attention_workspace(seqs, h, d, max_ctx, device)
+    ws.fill_(0xff)
+    vpa.paged_attention_plan(args[6], max_ctx, bt.shape[1], h, args[3], args[4], torch.bfloat16, ws)
+    header = ws[-256:].view(torch.int32)[:2].tolist()
+    cus = torch.cuda.get_device_properties(device).multi_processor_count
+
+    def items(chunk):
+        return int(np.sum((lens.astype(np.int64) + chunk - 1) // chunk))
+
+    short = max_ctx > 2048 and seqs * kvh <= 512 and (
+        items(1024) * kvh <= cus
+        or (lens.max() > 2048 and 8 * items(2048) * kvh > 9 * cus))
+    chunk = 1024 if short else 2048
+    assert header == [chunk.bit_length() - 1, items(chunk)]
+    out = vpa.paged_attention(*args, workspace=ws, planned=True)
+    torch.cuda.synchronize()
+    want = orc.paged_attention(q, kc, vc, bt, lens, max_ctx, d ** -0.5, dtype=orc.BF16)
+    assert_attention_close(orc.to_f32(to_host(out), orc.BF16), want, orc.BF16)
 
 
 @pytest.mark.parametrize("b,max_ctx,parts", [(1, 1, 0), (1, 129, 0), (3, 200, 0), (2, 256, 0),
