@@ -24,18 +24,27 @@
 namespace vpa {
 namespace {
 
-constexpr int kSmallWaves = 8;
 constexpr int kSmallMaxChunk = 1024;  // tokens, small_chunk_blocks' largest
+
+// Waves per workgroup: eight; four over 32-token blocks of eight 16-byte loads
+// per lane (16-bit head dim 128), which take more than 128 registers, so that
+// a CU could not hold two workgroups of eight, and of which a context of 512
+// tokens has only 16 (us per layer, eight -> four; sequences x tokens: 64 x
+// 13-38 10.1 -> 7.7, 64 x 77-128 11.8 -> 9.5, 8 x 154-256 7.6 -> 6.9, 8 x
+// 256-512 9.9 either way; the list form 7.2, 10.8, 7.1 and 9.4).
+template <typename C, int D, int BS>
+constexpr int kSmallWaves = BS == 32 && D * BS * (int)sizeof(C) / 1024 == 8 ? 4 : 8;
 
 // Tokens per wave: the largest chunk's share, and at least head_dim (the
 // merge reuses a wave's logits for its output).
-template <int D>
-constexpr int kSmallPT = D <= kSmallMaxChunk / kSmallWaves ? kSmallMaxChunk / kSmallWaves : D;
+template <int D, int NW>
+constexpr int kSmallPT = D <= kSmallMaxChunk / NW ? kSmallMaxChunk / NW : D;
 
 template <typename T, typename C, int D, int BS, int G>
 hipError_t launch_small_t(const DecodeArgs& a, const CacheGeom& g, const DecodeWorkspace& ws,
                           int target, hipStream_t stream) {
-  static_assert(kSmallPT<D> % 64 == 0 && kSmallPT<D> * kSmallWaves >= kSmallMaxChunk, "chunk");
+  constexpr int NW = kSmallWaves<C, D, BS>, PT = kSmallPT<D, NW>;
+  static_assert(PT % 64 == 0 && PT * NW >= kSmallMaxChunk, "chunk");
   // target > 0: at most `target` workgroups where the chunks are shorter than
   // the largest, else the largest chunks of every sequence
   const int64_t largest = std::max(1, (a.max_ctx + kSmallMaxChunk - 1) / kSmallMaxChunk);
@@ -46,7 +55,7 @@ hipError_t launch_small_t(const DecodeArgs& a, const CacheGeom& g, const DecodeW
   auto go = [&](auto kernel) {
     const DecodeAppend none{nullptr, nullptr, 0, 0};
     const DecodeAppend& app = a.append != nullptr ? *a.append : none;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)units), dim3(64 * kSmallWaves), 0, stream,
+    hipLaunchKernelGGL(kernel, dim3((unsigned)units), dim3(64 * NW), 0, stream,
                        static_cast<T*>(a.out), static_cast<const T*>(a.query),
                        static_cast<const C*>(a.key_cache), static_cast<const C*>(a.value_cache),
                        a.block_tables, a.block_table_stride, a.scale, a.num_heads,
@@ -61,9 +70,9 @@ hipError_t launch_small_t(const DecodeArgs& a, const CacheGeom& g, const DecodeW
   };
   if constexpr (!std::is_same_v<C, fp8_t> && fused_append_shape(D, BS)) {
     if (a.append != nullptr)
-      return go(paged_decode_rows_kernel<T, C, D, BS, G, kSmallPT<D>, kSmallWaves, true, true>);
+      return go(paged_decode_rows_kernel<T, C, D, BS, G, PT, NW, true, true>);
   }
-  return go(paged_decode_rows_kernel<T, C, D, BS, G, kSmallPT<D>, kSmallWaves, false, true>);
+  return go(paged_decode_rows_kernel<T, C, D, BS, G, PT, NW, false, true>);
 }
 
 template <typename T, typename C, int D, int BS>
@@ -127,6 +136,21 @@ hipError_t launch_small(int group, const DecodeArgs& a, const CacheGeom& g,
 // the list form, whose four-wave workgroups the dispatcher packs better, is
 // as fast or faster (24 x 700-1000 tokens 15.9 us there with 1024-token
 // chunks, 19.0 here; 16 x 13.9 and 14.7; 16 x 100-1500 15.9 and 13.4).
+//
+// Up to a maximum of 2048 tokens the list form is one launch once the step's
+// list is there, and this one always two. Per layer of a planned step (us,
+// list -> here; 16 heads over 8, head dim 128; maximum and the share of it
+// that the contexts fill): 1 sequence, 2048, 5-15 % 6.2 -> 8.0, 30-50 % 12.0
+// -> 9.1, half to all 18.0 -> 9.5; 1, 1024, 5.9 -> 7.6, 8.3 -> 9.0 and 10.7 ->
+// 9.2; 8, 1024, 6.5 -> 8.2, 9.2 -> 9.8 and 14.0 -> 10.7; 16, 1024, 6.7 -> 8.3,
+// 9.5 -> 10.9 and 14.9 -> 14.6. So a maximum frozen at more than about three
+// times the longest context costs up to 2 us, and one that a context fills to
+// the half or more, as the table widths of captured graphs do, gains as much
+// or more. Without a list (a call that would build its own first) this form
+// is the faster one throughout (1 sequence, 2048: 10.9, 16.7 and 22.8 -> 7.3,
+// 8.6 and 9.0). From 8 sequences of more than 4096 on, the same holds: worst
+// in a planned step where a CU gets one or two workgroups (8 x 3072-6144 31.1
+// -> 37.5, 8 x 300-900 14.8 -> 10.3, 16 x 4096-8192 72.3 -> 73.6).
 int decode_small_target(int num_seqs, int num_kv_heads, int max_ctx, int max_parts) {
   if (num_seqs > kSmallMaxSeqs) return -1;
   if (max_ctx <= 512) return 0;
