@@ -35,25 +35,44 @@ hipError_t split_block(const PrefillArgs& a, const CacheGeom& g, hipStream_t str
 
 }  // namespace
 
-// Up to one 128-row tile per four CUs, whose 32-row tiles then have a CU each,
-// unless a wave would get no more than half a tile of keys; up to one per two
-// CUs where the keys are many. Above, the tiles of 128 rows, which read each
-// K / V operand from L2 a quarter as often, fill the chip. Measured (us, 128-row
-// tiles -> split keys; bf16, 16 heads over 8, sequences x new over prior
-// tokens): 1 x 100 over 400 14.8 -> 10.9, 1 x 512 over 0 14.7 -> 12.0, over
-// 1500 37.4 -> 22.7, over 6000 116 -> 62 (26 GFLOP: 424 TFLOP/s), 1 x 1024
-// over 1024 35.7 -> 30.7, 2 x 512 over 512 21.3 -> 19.7; the other way round,
-// 1 x 16 over 0 5.9 -> 7.8, 4 x 200 over 0 10.1 -> 11.9, 4 x 400 over 400 20.2
-// -> 31.0; 32 heads over 4: 1 x 512 over 1500 45.9 -> 43.4, 1 x 1024 over 1024
-// 44.3 -> 52.5. Head dim 128, the decoder's, at 16- and 32-token blocks only.
+// Where the 32-row tiles get a CU each (a workgroup fills one: 128 KiB of
+// LDS) and there are enough keys that a wave's share pays for the merge.
+// Measured (us, 128-row tiles -> split keys; bf16, 16 heads over 8, sequences
+// x new over prior tokens): 1 x 100 over 400 14.8 -> 10.9, 1 x 512 over 0 14.7
+// -> 12.0, over 1500 37.4 -> 22.7, over 6000 116 -> 62 (26 GFLOP: 424 TFLOP/s),
+// 4 x 100 over 500 18.7 -> 13.4. Up to 64 rows, whose 128-row form runs half
+// its waves, need more than 192 keys (4 x 16 over 96 7.2 -> 7.6, 8 x 16 over
+// 176 7.8 -> 9.1, over 208 9.2 -> 9.1), and 384 from a tile per two CUs on (16
+// x 16 over 304 10.4 -> 11.2). fp8 caches and the groups at run time gain from
+// 64 keys on (fp8 4 x 8 over 88 6.2 -> 5.7).
+// With up to two 32-row tiles per CU some CUs serve two, and the 128-row
+// tiles, which read each K / V operand from L2 a quarter as often, win (4 x
+// 200 over 500 21.0 -> 25.2, 8 x 100 over 2000 47.7 -> 68.9, 2 x 512 over 0
+// 16.4 -> 17.0), but for one long causal chunk, whose last rows see far more
+// keys than its first (1 x 700 over 500 30.8 -> 26.1, 1 x 1024 over 500 37.2
+// -> 33.5; over 6000 143.9 -> 150), and the groups at run time (32 heads over
+// 4: 1 x 400 over 2000 77.1 -> 64.0, 4 x 100 over 500 25.7 -> 27.5).
+// Head dim 128, the decoder's, at 16- and 32-token blocks, is what is built: a
+// 16-bit cache's two stages of four tiles do not fit the LDS at head dims 192
+// and 256 (192 and 256 KiB); 64 and 96, 8-token blocks and the larger head
+// dims over fp8 caches have not been tried.
 bool prefill_split_keys(const PrefillArgs& a, const CacheGeom& g) {
   if (g.head_dim != 128 || g.block_size < 16) return false;
-  const int64_t tiles = prefill_row_tiles(a.max_query_len, a.num_heads / g.num_kv_heads,
-                                          kPrefillWaves * 32) *
-                        a.num_seqs * g.num_kv_heads;
+  const int group = a.num_heads / g.num_kv_heads;
+  const bool any_group = group != 1 && group != 2 && group != 4;
+  const int64_t pairs = (int64_t)a.num_seqs * g.num_kv_heads;
+  const int64_t tiles = prefill_row_tiles(a.max_query_len, group, 32) * pairs;
   const int64_t cus = device_cu_count();
-  return (tiles * 4 <= cus && a.max_kv_len > 2 * kPrefillKeys) ||
-         (tiles * 2 <= cus && a.max_kv_len >= 16 * kPrefillKeys);
+  if (tiles <= cus) {
+    const bool few_rows = (int64_t)a.max_query_len * group <= 64 && !any_group &&
+                          a.k_scale == nullptr;
+    return a.max_kv_len > (!few_rows ? 2 : 4 * tiles <= cus ? 6 : 12) * kPrefillKeys;
+  }
+  if (any_group)
+    return 2 * prefill_row_tiles(a.max_query_len, group, kPrefillWaves * 32) * pairs <= cus &&
+           a.max_kv_len >= 16 * kPrefillKeys;
+  return tiles <= 2 * cus && a.causal && a.max_query_len > 512 &&
+         a.max_kv_len < 4 * (int64_t)a.max_query_len;
 }
 
 hipError_t launch_prefill_split(int dtype, int cache_dtype, const PrefillArgs& a,

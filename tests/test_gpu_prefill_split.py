@@ -2,7 +2,7 @@
 dim 128): few row tiles, whose workgroups split a tile's keys over their
 waves, and the same sequences among enough others that they do not, against
 the fp64 oracle. Key counts on both sides of a tile (32), a step of four tiles
-(128) and the rule's 64 and 512."""
+(128) and the rule's 64 and, for at most 64 rows, 192."""
 
 import numpy as np
 import pytest
@@ -13,14 +13,19 @@ from tests.test_gpu_prefill_vector import vector_case
 
 pytestmark = pytest.mark.gpu
 
-# (prior, new) tokens; with 16 heads over 8, at most 64 tiles of 128 rows
+# (prior, new) tokens; with 16 heads over 8, at most 256 tiles of 32 rows but
+# for the last two
 FEW = {
     "one_token": ([600], [1]),
     "keys_65": ([0], [65]),
     "keys_64": ([0, 31], [64, 33]),
-    "ragged": ([0, 127, 513, 0], [129, 1, 31, 0]),
+    "few_rows_192": ([176, 100], [16, 3]),
+    "few_rows_193": ([177, 100], [16, 3]),
+    "ragged": ([0, 127, 513, 0], [128, 1, 31, 0]),
     "long": ([1000], [300]),
-    "many_keys": ([511, 300], [200, 260]),
+    "many_keys": ([511, 300], [200, 250]),
+    "two_per_cu": ([511, 300], [200, 260]),  # 272 tiles: not split
+    "two_per_cu_long": ([0], [528]),  # 264 tiles of one chunk: split where causal
 }
 
 
