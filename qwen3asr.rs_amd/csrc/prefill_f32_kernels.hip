@@ -13,8 +13,8 @@
 // Work unit: one wave, 32 rows, 32 keys per tile. v_mfma_f32_32x32x2_f32
 // multiplies and adds in f32, so nothing is held or computed in fewer bits
 // than on the vector ALUs. It takes 64 cycles for 256 bytes of each operand,
-// sixteen times the cycles per byte of the 16-bit instruction, which decides
-// the rest: the matrix pipes are what bounds this kernel, the operands can
+// eight times the cycles per byte of the 16-bit instruction (sixteen per
+// operation), which decides the rest: the matrix pipes are what bounds this kernel, the operands can
 // come straight from the caches, and no LDS tile, transpose or barrier is
 // needed. Both operands fall on the cache layouts: MFMA sums over k in any
 // order that A and B share, so
@@ -441,10 +441,19 @@ hipError_t launch_f32_t(const F32Args& a, const CacheGeom& g, hipStream_t stream
 // 8): 1 x 100 over 0 11 / 23, 1 x 512 over 6000 264 / 1035, 8 x 512 over 1000
 // 241 / 380, 64 x 512 over 512 1344 / 1473, 32 x 300 over 0 143 / 152; 32
 // heads over 4 with many short rows: 32 x 300 over 0 259 / 225, 64 x 64 over
-// 200 172 / 153.
+// 200 172 / 153. One tile of keys has nothing to split (64 x 1 over 31, head
+// dim 192 over fp8 30.0 / 25.0). Where a sequence has no more than 32 rows,
+// three of the four waves of the other form have none, and its LDS (all four
+// waves' queries) keeps workgroups off the CU: above head dim 64 that costs
+// more than the merge from two tiles of keys on (head dim 128, 128 x 1 over
+// 199 56 / 91; 192 over fp8, 128 x 1 over 63 58 / 84; but head dim 64, 128 x 1
+// over 95 20.9 / 16.3).
 bool split_keys(const F32Args& a, const CacheGeom& g) {
+  if (a.max_kv_len <= kFKeys) return false;
   const int64_t rows = (int64_t)a.max_query_len * (a.num_heads / g.num_kv_heads);
   const int64_t tiles = (rows + 4 * kFRows - 1) / (4 * kFRows) * a.num_seqs * g.num_kv_heads;
+  if (rows <= kFRows && g.head_dim > 64 && (a.max_kv_len > 2 * kFKeys || g.head_dim > 128))
+    return true;
   return a.max_kv_len > 10 * kFKeys || tiles < 4 * (int64_t)device_cu_count();
 }
 
@@ -497,6 +506,19 @@ hipError_t launch_prefill_f32(int dtype, int cache_dtype, void* out, const void*
                               int32_t causal, int32_t num_heads, const CacheGeom& g,
                               const float* k_scale, const float* v_scale, hipStream_t stream) {
   if (dtype != VPA_DTYPE_F32) return hipErrorInvalidValue;
+  // Over one tile of keys a wave here is a chain of D matrix instructions of
+  // 64 cycles, and where the vector kernel's workgroups have a CU each that is
+  // quicker (us, vector / here; 16 heads over 8, sequences x new over prior
+  // tokens: 1 x 1 over 0 8.8 / 9.7, 1 x 32 over 0 9.8 / 10.3; head dim 64, 1 x
+  // 16 over 0 5.9 / 7.0, 32 x 1 over 31 6.6 / 5.9; with more workgroups than
+  // CUs, head dim 128, 64 x 16 over 16 27.1 / 13.9)
+  if (max_kv_len <= kFKeys &&
+      prefill_vector_workgroups(num_seqs, max_query_len, num_heads / g.num_kv_heads,
+                                g.num_kv_heads) <= device_cu_count())
+    return launch_prefill_vector(dtype, cache_dtype, out, query, key_cache, value_cache,
+                                 block_tables, block_table_stride, cu_seqlens_q, context_lens,
+                                 num_seqs, max_query_len, max_kv_len, total_query_rows, scale,
+                                 denom_eps, causal, num_heads, g, k_scale, v_scale, stream);
   const F32Args a{static_cast<float*>(out), static_cast<const float*>(query), key_cache,
                   value_cache, block_tables, block_table_stride, cu_seqlens_q, context_lens,
                   num_seqs, max_query_len, max_kv_len, total_query_rows, scale, denom_eps,

@@ -4,7 +4,7 @@
 // head-dim / block-size pairs without a whole number of 1 KiB DMAs per tile,
 // with any number of query heads per kv head (the Metal dispatch takes
 // q_per_kv as a grid dimension, vasr-paged-attn/src/metal/kernels/
-// mod.rs:145-283).
+// mod.rs:145-283), and small f32 calls over at most 32 keys.
 //
 // Decode (paged_attention) runs the head-dim / block-size pairs its own
 // kernels do not take on this kernel too, f32 queries over fp8 caches among
@@ -347,19 +347,35 @@ hipError_t launch_vector_t(void* out, const void* query, const void* kc, const v
   return hipGetLastError();
 }
 
+// Head dims built for a query and cache type: every one for f32 queries; for
+// 16-bit ones those with a block size whose tiles are not whole 1 KiB DMAs
+// (96 at 8 tokens; fp8 64, 96 and 192 at 8 and 96 at 16), which neither the
+// MFMA prefill nor a decode kernel takes.
+constexpr bool vector_dim_built(bool f32, bool fp8, int d) {
+  if (f32) return d == 64 || d == 96 || d == 128 || d == 192 || d == 256;
+  return d == 96 || (fp8 && (d == 64 || d == 192));
+}
+
+template <typename T, typename C, int D, typename... A>
+hipError_t vector_one(A... args) {
+  if constexpr (vector_dim_built(std::is_same_v<T, float>, std::is_same_v<C, fp8_t>, D))
+    return launch_vector_t<T, C, D>(args...);
+  return hipErrorInvalidValue;
+}
+
 template <typename T, typename C, typename... A>
 hipError_t vector_dim(int d, A... args) {
   switch (d) {
     case 64:
-      return launch_vector_t<T, C, 64>(args...);
+      return vector_one<T, C, 64>(args...);
     case 96:
-      return launch_vector_t<T, C, 96>(args...);
+      return vector_one<T, C, 96>(args...);
     case 128:
-      return launch_vector_t<T, C, 128>(args...);
+      return vector_one<T, C, 128>(args...);
     case 192:
-      return launch_vector_t<T, C, 192>(args...);
+      return vector_one<T, C, 192>(args...);
     case 256:
-      return launch_vector_t<T, C, 256>(args...);
+      return vector_one<T, C, 256>(args...);
     default:
       return hipErrorInvalidValue;
   }
@@ -368,12 +384,10 @@ hipError_t vector_dim(int d, A... args) {
 }  // namespace
 
 bool prefill_vector_supported(int dtype, int cache_dtype, int head_dim, int block_size) {
-  const bool qt = dtype == VPA_DTYPE_F32 || dtype == VPA_DTYPE_BF16 || dtype == VPA_DTYPE_F16;
-  const bool ct = cache_dtype == dtype || cache_dtype == VPA_DTYPE_FP8_E4M3;
-  const bool dim = head_dim == 64 || head_dim == 96 || head_dim == 128 || head_dim == 192 ||
-                   head_dim == 256;
+  const bool f32 = dtype == VPA_DTYPE_F32, fp8 = cache_dtype == VPA_DTYPE_FP8_E4M3;
+  const bool qt = f32 || dtype == VPA_DTYPE_BF16 || dtype == VPA_DTYPE_F16;
   const bool blk = block_size == 8 || block_size == 16 || block_size == 32;
-  return qt && ct && dim && blk;
+  return qt && (cache_dtype == dtype || fp8) && blk && vector_dim_built(f32, fp8, head_dim);
 }
 
 int64_t prefill_vector_workgroups(int32_t num_seqs, int32_t max_query_len, int32_t group,
@@ -397,8 +411,7 @@ hipError_t launch_prefill_vector(int dtype, int cache_dtype, void* out, const vo
       cu_seqlens_q, context_lens, num_seqs, max_query_len, max_kv_len, total_query_rows, scale, \
       denom_eps, causal, num_heads, g, k_scale, v_scale, stream
   if (dtype == VPA_DTYPE_F32)
-    // (f32 caches: prefill_f32_kernels.hip, and every decode shape has a kernel)
-    return f8 ? vector_dim<float, fp8_t>(VPA_VEC_ARGS) : hipErrorInvalidValue;
+    return f8 ? vector_dim<float, fp8_t>(VPA_VEC_ARGS) : vector_dim<float, float>(VPA_VEC_ARGS);
   if (dtype == VPA_DTYPE_BF16)
     return f8 ? vector_dim<bf16_t, fp8_t>(VPA_VEC_ARGS)
               : vector_dim<bf16_t, bf16_t>(VPA_VEC_ARGS);

@@ -254,10 +254,10 @@ hipError_t launch_prefill_f32(int dtype, int cache_dtype, void* out, const void*
                               const float* k_scale, const float* v_scale, hipStream_t stream);
 
 // The vector-ALU prefill (prefill_vector_kernels.hip): the 16-bit shapes the
-// MFMA kernel does not take; also the decode of the head-dim / block-size
-// pairs no decode kernel takes (cu_seqlens_q null: one query per sequence).
-// Same arguments as launch_prefill_paged. (prefill_vector_supported names
-// the whole set, f32 prefills included, which launch_prefill_f32 serves.)
+// MFMA kernel does not take, and the f32 calls launch_prefill_f32 hands over;
+// also the decode of the head-dim / block-size pairs no decode kernel takes
+// (cu_seqlens_q null: one query per sequence). Same arguments as
+// launch_prefill_paged.
 bool prefill_vector_supported(int dtype, int cache_dtype, int head_dim, int block_size);
 int64_t prefill_vector_workgroups(int32_t num_seqs, int32_t max_query_len, int32_t group,
                                   int32_t num_kv_heads);

@@ -1,15 +1,17 @@
-"""GPU parity of the chunked prefill on the vector-ALU kernel against the fp64
-oracle: the configurations the MFMA kernel is not built for.
+"""GPU parity against the fp64 oracle of the chunked prefill's configurations
+next to the 16-bit kernel's 1, 2 and 4 query heads per kv head:
 
 * f32 queries over f32 caches and over fp8 caches with scales, the Metal
   prefill's `float` and `float, uint8_t` instances
   (prefill_paged_attn.metal:1606, 1610; F32 dispatch at
-  vasr-paged-attn/src/metal/kernels/mod.rs:119-137): rel 1e-5, causal
-  (flash varlen, eps 0) and not (the Metal kernel's 1e-6 and a large eps),
-  every head dim and block size, ragged lengths, absent blocks;
-* numbers of query heads per kv head the MFMA kernel does not take (3, 8,
-  16; the Metal dispatch takes any, mod.rs:145-283), 16-bit and fp8;
-* 16-bit and fp8 head-dim / block-size pairs without whole 1 KiB DMAs."""
+  vasr-paged-attn/src/metal/kernels/mod.rs:119-137), on the f32 matrix
+  instructions, and on the vector ALUs for at most 32 rows over 32 keys: rel
+  1e-5, causal (flash varlen, eps 0) and not (the Metal kernel's 1e-6 and a
+  large eps), every head dim and block size, ragged lengths, absent blocks;
+* other numbers of query heads per kv head (3, 8, 16; the Metal dispatch
+  takes any, mod.rs:145-283), 16-bit and fp8, on the 16-bit MFMA kernel;
+* 16-bit and fp8 head-dim / block-size pairs without whole 1 KiB DMAs, on the
+  vector ALUs."""
 
 import numpy as np
 import pytest
@@ -88,8 +90,8 @@ def test_prefill_f32_query_fp8_cache(device, d, bs, causal, scales):
 @pytest.mark.parametrize("h,kvh", [(24, 8), (64, 8), (16, 1), (32, 2), (8, 8)])
 @pytest.mark.parametrize("code", [orc.F32, orc.BF16, orc.F16])
 def test_prefill_query_heads_per_kv_head(device, h, kvh, code):
-    """3, 8 and 16 query heads per kv head (and 1 for f32) on the vector
-    kernel; 16-bit with 1 / 2 / 4 stays on the MFMA kernel."""
+    """3, 8 and 16 query heads per kv head (and 1), f32 on the f32 matrix
+    instructions and 16-bit on the 16-bit MFMA kernel."""
     got, want = vector_case(device, code, h, kvh, 128, 16, [7, 0, 260], [40, 65, 17],
                             seed=h + kvh + code)
     assert_attention_close(got, want, code, f"h={h} kvh={kvh} code={code}")
@@ -222,16 +224,62 @@ def test_prefill_any_group_infinite_values_and_zero_scale(device, code):
 
 
 @pytest.mark.parametrize("fp8", [False, True])
-@pytest.mark.parametrize("d,bs,n,prior", [(128, 16, 31, 70), (64, 32, 33, 5), (96, 8, 64, 129),
-                                          (192, 32, 20, 40), (256, 16, 34, 30)])
+@pytest.mark.parametrize("d,bs,n,prior", [(128, 16, 41, 70), (64, 32, 33, 5), (96, 8, 64, 129),
+                                          (192, 32, 40, 40), (256, 16, 34, 30)])
 def test_prefill_f32_many_short_rows(device, d, bs, n, prior, fp8):
-    """Many row tiles over at most 320 keys: a wave of the f32 kernel takes a
-    row tile of its own instead of a quarter of one tile's keys (the other
-    cases here have fewer than 1024 tiles, and split)."""
+    """Many row tiles over at most 320 keys, each sequence with more than 32
+    rows: a wave of the f32 kernel takes a row tile of its own instead of a
+    quarter of one tile's keys (the other cases here have fewer than 1024
+    tiles, and split)."""
     if fp8 and bs == 8:
         bs = 16
     b = 129
     rng = np.random.default_rng(n)
-    got, want = vector_case(device, orc.F32, 8, 8, d, bs, rng.integers(0, prior + 1, b),
-                            rng.integers(1, n + 1, b), seed=d + n, fp8=fp8)
+    new = rng.integers(1, n + 1, b)
+    new[0] = n
+    got, want = vector_case(device, orc.F32, 8, 8, d, bs, rng.integers(0, prior + 1, b), new,
+                            seed=d + n, fp8=fp8)
     assert_attention_close(got, want, orc.F32, f"d={d} bs={bs} fp8={fp8}")
+
+
+@pytest.mark.parametrize("h,kvh,n", [(24, 8, 20), (16, 8, 17), (33, 11, 64)])
+@pytest.mark.parametrize("causal,fp8", [(True, False), (False, False), (False, True)])
+def test_prefill_f32_many_short_rows_groups(device, h, kvh, n, causal, fp8):
+    """The same form with 2 and 3 query heads per kv head (row tiles that end
+    inside a position), without the causal mask, and with absent blocks. (The
+    fp8 codes have a standard deviation of 2; scales of 0.5 give scores and
+    values the unit deviation of the f32 cases. At 1 a score of deviation 2
+    alone rounds by about 2^-22, which times the largest value, 8, passes the
+    floor of the bound, 1e-5 * 0.03 * 8, at one of 20 million elements.)"""
+    b = 130
+    rng = np.random.default_rng(n + h)
+    prior, new = rng.integers(0, 90, b), rng.integers(1, n + 1, b)
+    prior[0], new[0] = 60, n
+
+    def absent(bt):
+        bt[0, 1] = 0xffffffff
+        bt[3, 0] = 1 << 30
+
+    got, want = vector_case(device, orc.F32, h, kvh, 128, 16, prior, new, seed=n, causal=causal,
+                            fp8=fp8, scales=(0.5, 0.5) if fp8 else (1.0, 1.0), mutate_bt=absent)
+    assert_attention_close(got, want, orc.F32, f"{h} over {kvh} causal={causal} fp8={fp8}")
+
+
+@pytest.mark.parametrize("d,bs", [(64, 16), (96, 32), (128, 8), (192, 16), (256, 32)])
+@pytest.mark.parametrize("h,kvh,n,keys", [(8, 8, 32, 32), (8, 8, 33, 33), (8, 8, 32, 33),
+                                          (16, 8, 16, 32), (16, 8, 17, 32), (24, 8, 1, 32),
+                                          (24, 8, 11, 31), (16, 8, 1, 1)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_prefill_f32_one_tile(device, d, bs, h, kvh, n, keys, fp8):
+    """Both sides of the line to the vector kernel: at most 32 rows over at
+    most 32 keys."""
+    if fp8 and bs == 8:
+        bs = 16
+
+    def absent(bt):
+        if bt.shape[1] > 1:
+            bt[0, 1] = 0xffffffff
+
+    got, want = vector_case(device, orc.F32, h, kvh, d, bs, [keys - n, 0, max(0, keys - n - 5)],
+                            [n, n, max(1, n - 1)], seed=d + n + keys, fp8=fp8, mutate_bt=absent)
+    assert_attention_close(got, want, orc.F32, f"d={d} n={n} keys={keys}")
