@@ -160,11 +160,28 @@ def test_fp8_decode_qwen3_asr_shape(device, code, bs):
 
 @pytest.mark.parametrize("bs", [16, 32])
 def test_fp8_decode_chunk_and_wave_boundaries(device, bs):
-    """Lengths at the per-wave (512-token) and per-chunk (2048-token)
-    boundaries of the rows kernel, merges of up to 4 chunks."""
+    """Lengths at the wave and chunk boundaries of the rows kernel's form for
+    few sequences (chunks of 1024 tokens here), merges of up to 8 chunks. (The
+    work list's: test_fp8_decode_on_the_list.)"""
     lens = [1, 511, 512, 513, 2047, 2048, 2049, 4095, 4096, 4097, 6145, 8191]
     got, want = fp8_decode_case(device, orc.BF16, 16, 8, 128, bs, lens, seed=200 + bs)
     assert_attention_close(got, want, orc.BF16, f"fp8 edges bs={bs}")
+
+
+@pytest.mark.parametrize("d,bs", [(64, 16), (64, 32), (128, 8), (128, 16), (128, 32), (96, 32),
+                                  (192, 16), (256, 8), (256, 16)])
+@pytest.mark.parametrize("code,h,long_chunks", [(orc.BF16, 16, False), (orc.F16, 16, True),
+                                                (orc.BF16, 32, True)])
+def test_fp8_decode_on_the_list(device, d, bs, code, h, long_chunks):
+    """More than 128 (sequence, kv head) pairs, which run over the work list,
+    at the 512-token waves and on both sides of its chunk lengths: 1024 tokens
+    where the items are no more than the compute units, 2048 where 24 further
+    sequences of 1100 tokens make them more."""
+    lens = [1, 511, 512, 513, 1023, 1024, 1025, 2047, 2048, 2049, 2600]
+    lens += [1100] * 24 if long_chunks else [5 + 9 * i for i in range(8)]
+    got, want = fp8_decode_case(device, code, h, 8, d, bs, lens, seed=d + bs + h,
+                                scales=(0.37, 3.1), planned=not long_chunks)
+    assert_attention_close(got, want, code, f"fp8 list d={d} bs={bs} h={h}")
 
 
 @pytest.mark.parametrize("factor", [2.0, 3.0, 10.0])

@@ -123,6 +123,36 @@ def test_fused_equals_two_calls(device, code, d, bs, h, kvh, planned):
     assert_attention_close(orc.to_f32(got, code), ref, code, f"fused d={d} bs={bs} h={h}")
 
 
+LIST_EDGES = [1, 2, 16, 17, 32, 511, 512, 513, 1023, 1024, 1025, 2047, 2048, 2049, 3000]
+
+
+@pytest.mark.parametrize("code,h,kvh,d,bs", [
+    (orc.F16, 16, 8, 128, 16), (orc.BF16, 32, 8, 128, 16), (orc.F16, 16, 4, 128, 32),
+    (orc.BF16, 16, 8, 64, 32), (orc.BF16, 16, 8, 96, 32), (orc.F16, 16, 8, 192, 16),
+    (orc.BF16, 8, 8, 256, 8), (orc.F16, 16, 4, 256, 16)])
+@pytest.mark.parametrize("many", [False, True])
+def test_fused_on_the_list_equals_two_calls(device, code, h, kvh, d, bs, many):
+    """The one-launch append inside the work-list form of the decode (EDGES
+    above are few enough for the form without one): more than 128 (sequence,
+    kv head) pairs, 48 sequences at most; with few further sequences the list
+    has 1024-token chunks, with many of 1100 tokens 2048-token ones."""
+    n = 48 if many else max(18, 136 // kvh)
+    rng = np.random.default_rng(d + h + 7 * code + many)
+    extra = n - len(LIST_EDGES)
+    lens = LIST_EDGES + ([1100] * extra if many else [int(x) for x in rng.integers(1, 200, extra)])
+    c = case(rng, code, h, kvh, d, bs, lens)
+    max_ctx, scale = int(c["lens"].max()), d ** -0.5
+    got, gk, gv = fused(device, c, code, max_ctx, scale, planned=many)
+    want, wk, wv = two_calls(device, c, code, bs, max_ctx, scale)
+    np.testing.assert_array_equal(gk, wk)
+    np.testing.assert_array_equal(gv, wv)
+    np.testing.assert_array_equal(got, want)
+    ref, rk, rv = oracle_fused(c, code, bs, max_ctx, scale)
+    np.testing.assert_array_equal(gk, rk)
+    np.testing.assert_array_equal(gv, rv)
+    assert_attention_close(orc.to_f32(got, code), ref, code, f"fused list d={d} bs={bs} h={h}")
+
+
 @pytest.mark.parametrize("what", ["bf16 batch 64", "f32", "fp8 cache", "head dim 96",
                                   "head dim 192"])
 def test_two_launch_form_equals_two_calls(device, what):

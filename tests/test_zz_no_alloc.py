@@ -109,6 +109,25 @@ def test_noalloc_equals_workspace_entry_point_twice(device, code, cache_code, d,
     assert_attention_close(orc.to_f32(got, code), ref, code, "noalloc second call")
 
 
+@pytest.mark.parametrize("code,cache_code", [(orc.BF16, orc.BF16), (orc.BF16, orc.FP8),
+                                             (orc.F32, orc.F32), (orc.F32, orc.FP8)])
+def test_noalloc_tight_layout(device, code, cache_code):
+    """A call whose caller workspace (128-token partitions) exceeds the 64 MiB
+    scratch, so that the scratch is laid out for the kernel's own partitions:
+    256 sequences, the longest 4600 tokens. Bit-equal to the workspace call
+    and checked against the oracle."""
+    rng = np.random.default_rng(5 + code + cache_code)
+    lens = [4600, 2049, 2048, 257, 256, 1] + [int(x) for x in rng.integers(1, 200, size=250)]
+    c = case(rng, code, lens, cache_code)
+    need = _lib.load().vpa_paged_attention_workspace_size(256, H, D, 4600)
+    assert need > 64 << 20
+    got = call(device, c, code, cache_code, True, 4600)
+    want = call(device, c, code, cache_code, False, 4600)
+    assert np.array_equal(got, want)
+    ref = orc.paged_attention(c["q"], c["kc"], c["vc"], c["bt"], c["lens"], 4600, D ** -0.5,
+                              dtype=code, kv_dtype=orc.FP8 if cache_code == orc.FP8 else None)
+    assert_attention_close(orc.to_f32(got, code), ref, code, "noalloc tight layout")
+
 
 def test_noalloc_calls_on_two_streams_are_ordered(device):
     """A large call on one stream and a small one on another, issued back to
