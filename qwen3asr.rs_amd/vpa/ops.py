@@ -48,12 +48,16 @@ def _err(msg: str):
     return VpaError(_lib.VPA_ERR_INVALID_ARGUMENT, msg)
 
 
+# a private name of torch's, absent from builds without a GPU
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(t: torch.Tensor) -> int:
     # the raw handle of torch.cuda.current_stream(t.device), without building
     # the Stream object around it on every call
-    if not t.is_cuda:
+    if _raw_stream is None or not t.is_cuda:
         return torch.cuda.current_stream(t.device).cuda_stream  # raises: not a GPU
-    return torch._C._cuda_getCurrentRawStream(t.get_device())
+    return _raw_stream(t.get_device())
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
