@@ -188,7 +188,8 @@ int vpa_paged_attention(void* out, const void* query, const float* k_scale,
  * every cache type); the workspace is that call's. Stream-ordered and
  * capture-safe; a no-op for configurations whose kernel never takes a list
  * (decodes of few sequences work their items out themselves; the list is
- * written for them too, for paged_cache_read).
+ * written for them too, for paged_cache_read). The chunk length of the list's
+ * items is chosen from the context lengths and is part of the list.
  * No counterpart in the reference (its decode kernel sizes its grid from
  * max_context_len only).
  */
@@ -293,7 +294,10 @@ int vpa_reshape_and_cache_paged_attention_planned(
  * whose layout does not
  * fit returns VPA_ERR_WORKSPACE (after the other argument checks, before
  * touching the device). Same arguments (minus the workspace), results and
- * errors as vpa_paged_attention. Every call on a GPU shares that GPU's
+ * errors as vpa_paged_attention (bit for bit, except where only the longest
+ * partitions fit and that call would take shorter ones, at most 512
+ * (sequence, kv head) pairs over contexts above 13000 tokens: there the split
+ * of the softmax rounds otherwise). Every call on a GPU shares that GPU's
  * array. Calls outside stream capture are ordered one after another on each
  * GPU (each call's stream waits for an event recorded after the previous
  * call, on whatever stream): several streams or threads do not race, their

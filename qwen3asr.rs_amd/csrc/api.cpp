@@ -379,12 +379,15 @@ int paged_attention_impl(void* out, const void* query, const float* k_scale,
                                               max_context_len, part_tokens);
   ws.planned = planned;
   // The append runs inside the decode launch (the rows kernel's fused form,
-  // 16-bit caches) for small batches only: measured on c3's length rule over
-  // 28 layers (us per step, two launches against one), batch 1: 214 / 142,
-  // 8: 363 / 284, 32: 741 / 672, and, with 2048-token chunks, 64: 1425-1459 / 1459, 128: 2437 / 2524,
-  // 256: 4484 / 4721. Inside a bandwidth-bound decode the token's sector
-  // writes interleave with the tile reads and cost more than the append's
-  // own launch; with few sequences that launch is what costs. Larger batches
+  // 16-bit caches) for small batches only: measured in a graph of 28 layers
+  // over geometric lengths around 800 tokens (us per step, two launches
+  // against one), batch 1 (450 tokens): 307 / 228, 8: 410 / 334, 32: 1009 /
+  // 932, 48: 1130 / 1065, 64: 1470 / 1391, 96: 1996 / 2000, 128: 2217 / 2224,
+  // 256: 4272 / 4450. (The bound of 48 was set where the two met with 2048-
+  // token chunks only; they meet between 64 and 96 now.) Inside a
+  // bandwidth-bound decode the token's sector writes interleave with the tile
+  // reads and cost more than the append's own launch; with few sequences that
+  // launch is what costs. Larger batches
   // and the other configurations run the append kernel on the derived slots,
   // then the decode: the same bytes and results either way.
   const bool fuse = append != nullptr &&

@@ -148,9 +148,10 @@ hipError_t launch_small(int group, const DecodeArgs& a, const CacheGeom& g,
 // the half or more, as the table widths of captured graphs do, gains as much
 // or more. Without a list (a call that would build its own first) this form
 // is the faster one throughout (1 sequence, 2048: 10.9, 16.7 and 22.8 -> 7.3,
-// 8.6 and 9.0). From 8 sequences of more than 4096 on, the same holds: worst
-// in a planned step where a CU gets one or two workgroups (8 x 3072-6144 31.1
-// -> 37.5, 8 x 300-900 14.8 -> 10.3, 16 x 4096-8192 72.3 -> 73.6).
+// 8.6 and 9.0). Longer contexts of 8 and more sequences are the other place
+// where a planned step can lose, worst with one or two workgroups per CU (8 x
+// 3072-6144 31.1 -> 37.5, 16 x 4096-8192 72.3 -> 73.6; but 8 x 300-900 14.8 ->
+// 10.3).
 int decode_small_target(int num_seqs, int num_kv_heads, int max_ctx, int max_parts) {
   if (num_seqs > kSmallMaxSeqs) return -1;
   if (max_ctx <= 512) return 0;
