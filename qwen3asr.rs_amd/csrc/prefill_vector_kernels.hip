@@ -261,12 +261,11 @@ __global__ __launch_bounds__(kVThreads) void prefill_paged_vector_kernel(
     const float s0 = visible(k0 + l) ? d0 * scale_log2 : -INFINITY;
     const float s1 = visible(k0 + l + 16) ? d1 * scale_log2 : -INFINITY;
     const float m_new = fmaxf(m, group16_max(fmaxf(s0, s1)));
-    float p0 = 0.f, p1 = 0.f, alpha = 1.f;
-    if (m_new != -INFINITY) {
-      alpha = m == -INFINITY ? 0.f : exp2f(m - m_new);
-      p0 = s0 == -INFINITY ? 0.f : exp2f(s0 - m_new);
-      p1 = s1 == -INFINITY ? 0.f : exp2f(s1 - m_new);
-    }
+    // the maximum drops a NaN, so a row of NaN scores (a NaN scale) still has
+    // -inf here: its probabilities are NaN all the same
+    const float alpha = m == -INFINITY ? 0.f : exp2f(m - m_new);
+    const float p0 = s0 == -INFINITY ? 0.f : exp2f(s0 - m_new);
+    const float p1 = s1 == -INFINITY ? 0.f : exp2f(s1 - m_new);
     lsum = lsum * alpha + group16_sum(p0 + p1);
     m = m_new;
     s_p[r][l] = p0;

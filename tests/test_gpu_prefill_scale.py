@@ -19,9 +19,27 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("h,kvh,d,bs", [(8, 8, 128, 16), (16, 8, 128, 16), (16, 4, 64, 32),
                                         (12, 4, 128, 32), (8, 4, 192, 16)])
 def test_nan_scale_gives_nan(device, code, fp8, h, kvh, d, bs):
-    rng = np.random.default_rng(d + h)
     # one sequence of many keys, a short one, one without a key
-    lens, new = [300, 7, 0], [40, 7, 2]
+    check_nan_scale(device, code, fp8, h, kvh, d, bs, [300, 7, 0], [40, 7, 2])
+
+
+@pytest.mark.parametrize("code", [orc.BF16, orc.F16, orc.F32])
+@pytest.mark.parametrize("h,kvh,d,bs", [(16, 8, 128, 16), (6, 2, 64, 32)])
+def test_nan_scale_over_few_keys(device, code, h, kvh, d, bs):
+    """At most 32 keys: f32 queries on the vector kernel."""
+    for fp8 in (False, True):
+        check_nan_scale(device, code, fp8, h, kvh, d, bs, [32, 7, 0], [5, 7, 2])
+
+
+@pytest.mark.parametrize("code,fp8,d,bs", [(orc.BF16, False, 96, 8), (orc.F16, False, 96, 8),
+                                           (orc.BF16, True, 64, 8), (orc.F16, True, 96, 16)])
+def test_nan_scale_without_whole_tiles(device, code, fp8, d, bs):
+    """The 16-bit queries' shapes on the vector kernel, over several tiles."""
+    check_nan_scale(device, code, fp8, 8, 4, d, bs, [70, 7, 0], [9, 7, 2])
+
+
+def check_nan_scale(device, code, fp8, h, kvh, d, bs, lens, new):
+    rng = np.random.default_rng(d + h)
     nb = 48
     if fp8:
         x = 16
@@ -42,5 +60,6 @@ def test_nan_scale_gives_nan(device, code, fp8, h, kvh, d, bs):
                 u32(cu, device), k_scale, one, scale, 1.0, causal=causal)
             torch.cuda.synchronize()
             got = orc.to_f32(to_host(out), code)
-            assert np.all(np.isnan(got[:47])), f"scale {scale} causal={causal}"
-            assert not np.any(got[47:])
+            rows = sum(new) - new[-1]  # the last sequence has no key
+            assert np.all(np.isnan(got[:rows])), f"scale {scale} causal={causal}"
+            assert not np.any(got[rows:])
