@@ -14,9 +14,10 @@
 // multiplies and adds in f32, so nothing is held or computed in fewer bits
 // than on the vector ALUs. It takes 64 cycles for 256 bytes of each operand,
 // eight times the cycles per byte of the 16-bit instruction (sixteen per
-// operation), which decides the rest: the matrix pipes are what bounds this kernel, the operands can
-// come straight from the caches, and no LDS tile, transpose or barrier is
-// needed. Both operands fall on the cache layouts: MFMA sums over k in any
+// operation), which decides the rest: the matrix pipes are what bounds this
+// kernel (busy 63 % of the time a SIMD has a wave, and for 18 % of the call it
+// has none; 8 sequences of 64-512 new over 0-1024 tokens), the operands can come
+// straight from the caches, and no LDS tile, transpose or barrier is needed. Both operands fall on the cache layouts: MFMA sums over k in any
 // order that A and B share, so
 //   S^T = K . Q^T   lane l holds key l % 32; its half h = l / 32 takes the
 //     16-byte units 2 i + h of the key row [D/4][BS][4], four MFMAs per unit

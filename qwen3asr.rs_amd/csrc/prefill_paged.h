@@ -293,7 +293,9 @@ constexpr int prefill_waves_per_eu() {
 // heads-fastest, so a group that does not divide 32 still fills every row of
 // a wave, and keeps the probabilities' f32 bits (f16: 22 of them), as the
 // vector kernel these groups ran on did: P goes through the P.V MFMAs as three
-// values of bf16 or two of f16 (take_part). MFMA-bound like the fixed groups.
+// values of bf16 or two of f16 (take_part). Bound by instruction issue like the
+// fixed groups (MFMAs busy 38 % and VALU active 44 % of the time a SIMD has a
+// wave), and by a ragged batch's tail (38 % of the call below without one).
 // Measured with the append before it (32 query over 4 kv heads, 12 sequences
 // of 33-450 new over 0-700 prior tokens, 21.2 GFLOP): f16 58.7 us, against 766
 // us on the vector kernel; error against 64 bits 2.07e-4 both ways, the
@@ -465,11 +467,10 @@ __attribute__((amdgpu_waves_per_eu(prefill_waves_per_eu<D>()))) void prefill_pag
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
     for (int e = 0; e < 16; ++e) o[dt][e] = 0.f;
-  // (never 0: a masked score is -inf, and 0 * -inf would be NaN; by a
-  // comparison, which is false for a NaN scale and keeps it, where fmaxf
-  // would drop it and leave the plain mean of the values)
-  const float abs_scale = fabsf(scale_log2);
-  const float sl = abs_scale < 1.17549435e-38f ? 1.17549435e-38f : abs_scale;
+  // (never 0: a masked score is -inf, and 0 * -inf would be NaN; at least the
+  // smallest normal value, by the bit patterns, whose order has a NaN scale on
+  // top: fmaxf would drop it and leave the plain mean of the values)
+  const float sl = __uint_as_float(max(__float_as_uint(fabsf(scale_log2)), 0x00800000u));
   float m = -INFINITY;   // reference max of the row (moves lazily), log2 units
   float mt = -INFINITY;  // the row's true max so far, log2 units
   float lsum = 0.f;      // this lane's share of the row's exp sum
