@@ -425,11 +425,10 @@ __global__ __launch_bounds__(64) void paged_decode_kernel(
 //
 // Work list: decode_plan_kernel (one workgroup) turns context_lens into the
 // list of (sequence, chunk) items, longest first, a chunk being at most NW *
-// PT tokens (list_chunk, plan_short_chunks), and a small header {log2 of the
-// chunk, item count}. All of it lives in the caller's workspace and is rebuilt
-// by every call, so the launches can be captured in a graph and replayed with
-// new lengths; max_context_len only sizes the grid, surplus workgroups exit at
-// once.
+// PT tokens (list_chunk), and a small header {log2 of the chunk, item count}. All of it lives in the caller's
+// workspace and is rebuilt by every call, so the launches can be captured
+// in a graph and replayed with new lengths; max_context_len only sizes the
+// grid, surplus workgroups exit at once.
 //
 // paged_decode_rows_kernel: one workgroup of NW waves per (item, kv head);
 // the chunk's blocks are split evenly over the waves (up to PT tokens each).
@@ -686,7 +685,7 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(
     part_tokens = block_size * small_chunk_blocks((max(L, 0) + block_size - 1) / block_size,
                                                   num_seqs, num_kv_heads, small_target,
                                                   block_size);
-  } else if (part_tokens < kDecodeChunk) {
+  } else {
     // (a list built by an earlier call is only trusted within this call's
     // bounds: no more parts than the workspace holds)
     part_tokens = max(part_tokens, 1 << min(queue[0], (uint32_t)__builtin_ctz(kDecodeChunk)));
