@@ -188,8 +188,7 @@ int vpa_paged_attention(void* out, const void* query, const float* k_scale,
  * every cache type); the workspace is that call's. Stream-ordered and
  * capture-safe; a no-op for configurations whose kernel never takes a list
  * (decodes of few sequences work their items out themselves; the list is
- * written for them too, for paged_cache_read). The chunk length of the list's
- * items is chosen from the context lengths and is part of the list.
+ * written for them too, for paged_cache_read).
  * No counterpart in the reference (its decode kernel sizes its grid from
  * max_context_len only).
  */

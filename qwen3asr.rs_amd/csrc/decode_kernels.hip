@@ -425,10 +425,10 @@ __global__ __launch_bounds__(64) void paged_decode_kernel(
 //
 // Work list: decode_plan_kernel (one workgroup) turns context_lens into the
 // list of (sequence, chunk) items, longest first, a chunk being at most NW *
-// PT tokens (list_chunk), and a small header {log2 of the chunk, item count}. All of it lives in the caller's
-// workspace and is rebuilt by every call, so the launches can be captured
-// in a graph and replayed with new lengths; max_context_len only sizes the
-// grid, surplus workgroups exit at once.
+// PT tokens (list_chunk), and a small header {log2 of the chunk, item count}.
+// All of it lives in the caller's workspace and is rebuilt by every call, so
+// the launches can be captured in a graph and replayed with new lengths;
+// max_context_len only sizes the grid, surplus workgroups exit at once.
 //
 // paged_decode_rows_kernel: one workgroup of NW waves per (item, kv head);
 // the chunk's blocks are split evenly over the waves (up to PT tokens each).
@@ -469,25 +469,10 @@ __device__ __forceinline__ int plan_bucket(int L, int p, int part_tokens) {
   return (int)(((int64_t)(part_tokens - n) * kPlanBuckets) / part_tokens);
 }
 
-// Whether a list takes the shorter of its two chunk lengths (1024 tokens):
-// where its items are no more than the CUs, or where the longer (2048) would
-// neither do for every context nor give a CU about one item each. Between,
-// some CUs get two of the shorter ones where each would get one of the longer,
-// and partial rows are written for contexts that fit one longer chunk. Us per
-// layer of a planned step, 16 heads over 8, head dim 128, shorter -> longer:
-// 24 x 1228-2048 tokens 34.4 -> 30.9, 20 x 200-4096 35.1 -> 32.8, 64 x 400-1228
-// 41.2 -> 38.8 (but 32 x 1228-2048 at head dim 64 24.0 -> 25.6, over fp8 18.6 ->
-// 23.7: the choice is the same for every cache type); the other way round, 24 x
-// 2048-4096 54.9 -> 59.7, 20 x 100-2048 19.4 -> 24.9.
-__device__ __forceinline__ bool plan_short_chunks(int64_t short_items, int64_t long_items,
-                                                  bool beyond, int cus) {
-  return short_items <= cus || (beyond && 8 * long_items > 9 * (int64_t)cus);
-}
-
 __global__ __launch_bounds__(1024) void decode_plan_kernel(
     const uint32_t* __restrict__ context_lens, int32_t num_seqs, int32_t max_ctx,
-    int32_t cap_tokens, int32_t part_tokens, int32_t max_part_tokens, int32_t num_kv_heads,
-    int32_t cus, uint2* __restrict__ items, uint32_t* __restrict__ queue) {
+    int32_t cap_tokens, int32_t part_tokens, uint2* __restrict__ items,
+    uint32_t* __restrict__ queue) {
   constexpr int NB = kPlanBuckets;
   __shared__ uint32_t s_wave[16][NB];
   __shared__ uint32_t s_base[NB + 1];
@@ -496,22 +481,6 @@ __global__ __launch_bounds__(1024) void decode_plan_kernel(
   const int per = (num_seqs + 1023) / 1024;
   const int s0 = min(tid * per, num_seqs);
   const int s1 = min(s0 + per, num_seqs);
-  // the chunk length, where the host leaves a choice (list_chunk): from the
-  // items that each of the two gives. Every wave counts them for itself, 64
-  // sequences at a time (there are at most 512), so no barrier is needed.
-  if (part_tokens != max_part_tokens) {
-    int nshort = 0, nlong = 0;
-    bool beyond = false;
-    for (int s = lane; s < num_seqs; s += 64) {
-      const int L = clamp_context(context_lens[s], max_ctx, cap_tokens);
-      nshort += L > 0 ? (L + part_tokens - 1) / part_tokens : 1;
-      nlong += L > 0 ? (L + max_part_tokens - 1) / max_part_tokens : 1;
-      beyond |= L > max_part_tokens;
-    }
-    if (!plan_short_chunks((int64_t)wave_sum_i32(nshort) * num_kv_heads,
-                           (int64_t)wave_sum_i32(nlong) * num_kv_heads, __any(beyond), cus))
-      part_tokens = max_part_tokens;
-  }
   uint32_t cnt[NB];
 #pragma unroll
   for (int b = 0; b < NB; ++b) cnt[b] = 0;
@@ -642,16 +611,21 @@ static_assert(kRowsPT >= kDecodeMinPartitionTokens && kF8PT >= kDecodeMinPartiti
 constexpr int kDecodeChunk = kRowsPT * kRowsWaves;
 static_assert(kF8PT * kF8Waves == kDecodeChunk, "one work list serves every cache type");
 
-// Tokens per work item, at least: half the largest chunk up to 512 (sequence,
-// kv head) pairs, where the longest item is the tail (us per layer, bf16,
-// 2048-token chunks -> 1024; 32 sequences geometric around 800 tokens 30.8 ->
-// 21.5, 64 48.3 -> 44.9; 32 x 3000-4000 77.4 -> 76.5) and the plan chooses
-// between the two from the lengths (plan_short_chunks), the largest above (256
-// x geometric 158.6 -> 165.7) and where it makes the merge launch unnecessary
-// (32 x 100-1500 with appends 26.1 -> 26.7). From host values that the plan
-// and the decode calls of a step share, for their grids (num_kv_heads:
-// replicas included; a workspace laid out for the largest chunk only,
-// max_parts, keeps that); the chunk itself is in the list's header.
+// Tokens per work item: half the largest chunk up to 512 (sequence, kv head)
+// pairs, where the longest item is the tail (us per layer, bf16, 2048-token
+// chunks -> 1024; 32 sequences geometric around 800 tokens 30.8 -> 21.5, 64
+// 48.3 -> 44.9; 32 x 3000-4000 77.4 -> 76.5), the largest above (256 x
+// geometric 158.6 -> 165.7) and where it makes the merge launch unnecessary
+// (32 x 100-1500 with appends 26.1 -> 26.7). Over 418 batches of up to 512
+// pairs (uniform, geometric and skewed lengths; bf16, fp8, head dim 64) the
+// shorter are 1 % off the better of the two on average and 11 % at worst (a
+// context just above 1024 gets a partial row and a second workgroup: 18 x
+// 200-4096 31.3 -> 34.3, 24 x 1228-2048 29.8 -> 31.6), the longer 10 % and 58 %
+// (two of 4000 among 24 26.6 -> 17.9). Choosing in the plan kernel by the
+// numbers of items was 4 % and 54 % off: the longest item decides as much.
+// From host values that the plan, the decode and the read-ceiling calls of a
+// step share (num_kv_heads: replicas included; a workspace laid out for the
+// largest chunk only, max_parts, keeps that).
 int list_chunk(int num_seqs, int num_kv_heads, int max_ctx, int max_parts) {
   constexpr int kHalf = kDecodeChunk / 2;
   return max_ctx > kDecodeChunk && (int64_t)num_seqs * num_kv_heads <= 512 &&
@@ -674,7 +648,7 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(
     T* __restrict__ out, const uint32_t* __restrict__ context_lens, int32_t num_seqs,
     int32_t max_ctx, int32_t cap_tokens, int32_t part_tokens, int32_t num_heads,
     const float* __restrict__ part, int32_t max_parts, int32_t small_target,
-    int32_t num_kv_heads, int32_t block_size, const uint32_t* __restrict__ queue) {
+    int32_t num_kv_heads, int32_t block_size) {
   constexpr int DPL = (D + 63) / 64;  // output elements per lane (the last partly, at D 96)
   constexpr int RS = kPartRow<D>;
   constexpr int R = kMergeRows;
@@ -685,10 +659,6 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(
     part_tokens = block_size * small_chunk_blocks((max(L, 0) + block_size - 1) / block_size,
                                                   num_seqs, num_kv_heads, small_target,
                                                   block_size);
-  } else {
-    // (a list built by an earlier call is only trusted within this call's
-    // bounds: no more parts than the workspace holds)
-    part_tokens = max(part_tokens, 1 << min(queue[0], (uint32_t)__builtin_ctz(kDecodeChunk)));
   }
   for (uint32_t u = blockIdx.x; u < units; u += gridDim.x) {
     const int s = (int)(u / (uint32_t)num_heads);
@@ -737,8 +707,8 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(
   }
 }
 
-// Merge of the partial rows of the list's chunks, of at least part_tokens
-// tokens (or, with small_target, of the small-grid form's).
+// Merge of the partial rows of chunks of part_tokens tokens (or, with
+// small_target, of the small-grid form's).
 template <typename T, int D>
 hipError_t launch_merge_t(void* out, const uint32_t* cl, int32_t num_seqs, int32_t max_ctx,
                           int32_t cap_tokens, int part_tokens, int32_t num_heads,
@@ -750,7 +720,7 @@ hipError_t launch_merge_t(void* out, const uint32_t* cl, int32_t num_seqs, int32
   hipLaunchKernelGGL((decode_merge_kernel<T, D>), dim3((unsigned)waves), dim3(64), 0, stream,
                      static_cast<T*>(out), cl, num_seqs, max_ctx, cap_tokens, part_tokens,
                      num_heads, ws.part_out, ws.max_parts, small_target, g.num_kv_heads,
-                     g.block_size, ws.queue);
+                     g.block_size);
   return hipGetLastError();
 }
 
@@ -784,8 +754,7 @@ hipError_t launch_decode_rows_c(void* out, const void* q, const void* kc, const 
   hipError_t e = hipSuccess;
   if (!ws.planned) {
     hipLaunchKernelGGL(decode_plan_kernel, dim3(1), dim3(1024), 0, stream, cl, num_seqs,
-                       max_ctx, cap_tokens, chunk, kDecodeChunk, g.num_kv_heads,
-                       device_cu_count(), ws.items, ws.queue);
+                       max_ctx, cap_tokens, chunk, ws.items, ws.queue);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
@@ -1038,7 +1007,8 @@ __global__ __launch_bounds__(64 * kRowsWaves) void paged_read_kernel(
     const uint32_t* __restrict__ block_tables, int32_t block_table_stride,
     int32_t num_kv_heads, int64_t num_blocks, int64_t block_stride_v, int64_t head_stride_v,
     const uint2* __restrict__ items, const uint32_t* __restrict__ queue, int32_t num_seqs,
-    int32_t max_ctx, int32_t cap_tokens, uint32_t magic, uint32_t* __restrict__ sink) {
+    int32_t max_ctx, int32_t cap_tokens, uint32_t magic, uint32_t* __restrict__ sink,
+    int32_t chunk_blocks) {
   constexpr int NW = kRowsWaves;
   constexpr int NV = VPA_READ_NV;    // loads per lane per stage
   const int lane = threadIdx.x & 63;
@@ -1046,14 +1016,13 @@ __global__ __launch_bounds__(64 * kRowsWaves) void paged_read_kernel(
   const uint32_t w = blockIdx.x;
   const int j = (int)(w % (uint32_t)num_kv_heads);
   const uint32_t want = w / (uint32_t)num_kv_heads;
-  const uint32_t chunk_log2 = queue[0], nitems = queue[1];
+  const uint32_t nitems = queue[1];
   const uint2 item = items[want];
   asm volatile("" ::"s"(nitems), "s"(item.x), "s"(item.y));
   if (want >= nitems) return;
   const int s = (int)(item.x >> 16);
   const int chunk = (int)(item.x & 0xffffu);
   if (s >= num_seqs) return;
-  const int chunk_blocks = max(1, (1 << min(chunk_log2, (uint32_t)__builtin_ctz(kDecodeChunk))) / BS);
   const int L = clamp_context(item.y, max_ctx, cap_tokens);
   if (L <= 0) return;
   const int nblk = (L + BS - 1) / BS;
@@ -1115,7 +1084,7 @@ hipError_t launch_read_t(const void* kc, const void* vc, const uint32_t* bt, int
                      0, stream, static_cast<const uint4*>(kc), static_cast<const uint4*>(vc), bt,
                      bts, g.num_kv_heads, g.num_blocks, g.block_stride / per_vec,
                      g.head_stride / per_vec, ws.items, ws.queue, num_seqs, max_ctx,
-                     bts * g.block_size, magic, sink);
+                     bts * g.block_size, magic, sink, chunk / BS);
   return hipGetLastError();
 }
 
@@ -1157,7 +1126,7 @@ hipError_t launch_decode_plan(int dtype, const uint32_t* context_lens, int32_t m
   hipLaunchKernelGGL(decode_plan_kernel, dim3(1), dim3(1024), 0, stream, context_lens, num_seqs,
                      max_context_len, block_table_stride * g.block_size,
                      list_chunk(num_seqs, g.num_kv_heads * g.kv_rep, max_context_len, ws.max_parts),
-                     kDecodeChunk, g.num_kv_heads * g.kv_rep, device_cu_count(), ws.items,
+                     ws.items,
                      ws.queue);
   return hipGetLastError();
 }

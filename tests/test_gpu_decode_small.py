@@ -3,8 +3,8 @@ list, chunk length worked out on the device) and of the work list's two chunk
 lengths, against the fp64 oracle, at the sizes where each takes over: one
 chunk up to a maximum of 512 tokens; chunks of 256, 512 and 1024 tokens up to
 128 (sequence, kv head) pairs; above, the list, with 2048-token chunks, or
-1024-token ones where the maximum exceeds 2048, there are at most 512 pairs
-and the lengths ask for it. Lengths sit on both sides of tiles and chunks,
+1024-token ones where the maximum exceeds 2048 and there are at most 512
+pairs. Lengths sit on both sides of tiles and chunks,
 with empty contexts, absent blocks and a maximum (as frozen in a captured
 graph) above every length. The list's cases have enough sequences for it at
 every number of kv heads here."""
@@ -32,7 +32,7 @@ CASES = {
     "list_1024": ([600 + 91 * i for i in range(16)] + [1024, 2048, 0] + [90] * 21, 2200),
     "list_one_chunk": ([130 + 5 * i for i in range(40)], 1024),
     "list_2048": ([(53 * i) % 700 for i in range(64)] + [2048, 2049], 2049),
-    "list_2048_choice": ([1100 + 37 * i for i in range(24)] + [1024, 1] + [300] * 8, 4096),
+    "list_1024_full": ([1100 + 37 * i for i in range(24)] + [1024, 1] + [300] * 8, 4096),
 }
 
 
@@ -101,20 +101,14 @@ def test_decode_small_grid_append(device, name, h, kvh, d, bs):
 
 
 @pytest.mark.parametrize("seqs,kvh,lo,hi,max_ctx", [
-    (40, 8, 1, 700, 4096),     # 1024-token items no more than the CUs
-    (24, 8, 1228, 2048, 4096),  # twice as many items of 1024 as of 2048, which fit the CUs
-    (17, 8, 200, 4096, 4096),
-    (60, 8, 1000, 4096, 4096),  # more items than CUs either way, some beyond 2048
-    (64, 8, 400, 1228, 8192),  # none beyond 2048
-    (24, 8, 1228, 2048, 2048),  # no choice: one chunk reaches the maximum
-    (65, 8, 1, 4096, 4096),    # no choice: more than 512 pairs
+    (24, 8, 1228, 2048, 4096), (64, 8, 400, 2049, 2049),
+    (24, 8, 1228, 2048, 2048),  # one chunk reaches the maximum
+    (65, 8, 1, 4096, 4096),     # more than 512 pairs
     (200, 1, 900, 3000, 3000)])
-def test_list_chunk_length_follows_the_items(device, seqs, kvh, lo, hi, max_ctx):
-    """The list's header: log2 of its chunk length and the number of items,
-    against the rule worked out here (1024-token chunks where they are no
-    more items than compute units, or where some context exceeds 2048 tokens
-    and 2048-token chunks are more than 9/8 of the units; else 2048), and the
-    decode over it against the oracle."""
+def test_list_chunk_length(device, seqs, kvh, lo, hi, max_ctx):
+    """The list's header: log2 of its chunk length and the number of items
+    (1024-token chunks above 2048 tokens for up to 512 pairs, else 2048), and
+    the decode over it against the oracle."""
     h, d, bs = 2 * kvh, 64, 16
     rng = np.random.default_rng(seqs + hi)
     lens = rng.integers(lo, hi, size=seqs, endpoint=True)
@@ -128,16 +122,9 @@ def test_list_chunk_length_follows_the_items(device, seqs, kvh, lo, hi, max_ctx)
     ws.fill_(0xff)
     vpa.paged_attention_plan(args[6], max_ctx, bt.shape[1], h, args[3], args[4], torch.bfloat16, ws)
     header = ws[-256:].view(torch.int32)[:2].tolist()
-    cus = torch.cuda.get_device_properties(device).multi_processor_count
-
-    def items(chunk):
-        return int(np.sum((lens.astype(np.int64) + chunk - 1) // chunk))
-
-    short = max_ctx > 2048 and seqs * kvh <= 512 and (
-        items(1024) * kvh <= cus
-        or (lens.max() > 2048 and 8 * items(2048) * kvh > 9 * cus))
-    chunk = 1024 if short else 2048
-    assert header == [chunk.bit_length() - 1, items(chunk)]
+    chunk = 1024 if max_ctx > 2048 and seqs * kvh <= 512 else 2048
+    assert header == [chunk.bit_length() - 1,
+                      int(np.sum((lens.astype(np.int64) + chunk - 1) // chunk))]
     out = vpa.paged_attention(*args, workspace=ws, planned=True)
     torch.cuda.synchronize()
     want = orc.paged_attention(q, kc, vc, bt, lens, max_ctx, d ** -0.5, dtype=orc.BF16)

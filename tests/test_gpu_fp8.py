@@ -175,10 +175,9 @@ def test_fp8_decode_chunk_and_wave_boundaries(device, bs):
 def test_fp8_decode_on_the_list(device, d, bs, code, h, long_chunks):
     """More than 128 (sequence, kv head) pairs, which run over the work list,
     at the 512-token waves and on both sides of its chunk lengths: 1024 tokens
-    where the items are no more than the compute units, 2048 where 24 further
-    sequences of 1100 tokens make them more."""
+    up to 512 pairs, 2048 where 54 further sequences make them more."""
     lens = [1, 511, 512, 513, 1023, 1024, 1025, 2047, 2048, 2049, 2600]
-    lens += [1100] * 24 if long_chunks else [5 + 9 * i for i in range(8)]
+    lens += [20] * 54 if long_chunks else [5 + 9 * i for i in range(8)]
     got, want = fp8_decode_case(device, code, h, 8, d, bs, lens, seed=d + bs + h,
                                 scales=(0.37, 3.1), planned=not long_chunks)
     assert_attention_close(got, want, code, f"fp8 list d={d} bs={bs} h={h}")

@@ -134,8 +134,8 @@ LIST_EDGES = [1, 2, 16, 17, 32, 511, 512, 513, 1023, 1024, 1025, 2047, 2048, 204
 def test_fused_on_the_list_equals_two_calls(device, code, h, kvh, d, bs, many):
     """The one-launch append inside the work-list form of the decode (EDGES
     above are few enough for the form without one): more than 128 (sequence,
-    kv head) pairs, 48 sequences at most; with few further sequences the list
-    has 1024-token chunks, with many of 1100 tokens 2048-token ones."""
+    kv head) pairs, 48 sequences at most; few further sequences, or many of
+    1100 tokens, each then of two chunks."""
     n = 48 if many else max(18, 136 // kvh)
     rng = np.random.default_rng(d + h + 7 * code + many)
     extra = n - len(LIST_EDGES)
