@@ -381,9 +381,9 @@ int paged_attention_impl(void* out, const void* query, const float* k_scale,
   // The append runs inside the decode launch (the rows kernel's fused form,
   // 16-bit caches) for small batches only: measured in a graph of 28 layers
   // over geometric lengths around 800 tokens (us per step, two launches
-  // against one), batch 1 (450 tokens): 307 / 228, 8: 410 / 334, 32: 1009 /
-  // 932, 48: 1130 / 1065, 64: 1470 / 1391, 96: 1996 / 2000, 128: 2217 / 2224,
-  // 256: 4272 / 4450. (The bound of 48 was set where the two met with 2048-
+  // against one), batch 1 (450 tokens): 306 / 226, 8: 411 / 332, 32: 774 /
+  // 709, 48: 1119 / 1060, 64: 1456 / 1386, 96: 1988 / 2001, 128: 2207 / 2229,
+  // 256: 4263 / 4446. (The bound of 48 was set where the two met with 2048-
   // token chunks only; they meet between 64 and 96 now.) Inside a
   // bandwidth-bound decode the token's sector writes interleave with the tile
   // reads and cost more than the append's own launch; with few sequences that
