@@ -52,6 +52,13 @@ hipError_t split_block(const PrefillArgs& a, const CacheGeom& g, hipStream_t str
 // keys than its first (1 x 700 over 500 30.8 -> 26.1, 1 x 1024 over 500 37.2
 // -> 33.5; over 6000 143.9 -> 150), and the groups at run time (32 heads over
 // 4: 1 x 400 over 2000 77.1 -> 64.0, 4 x 100 over 500 25.7 -> 27.5).
+// Those batches were of equal queries and contexts. Where they differ, one
+// sequence's rows are what is left at the end, and the split form gains far
+// more than it costs an equal batch: over 6000 / 800 tokens 256 + 3 x 16 rows of
+// an fp8 cache 119 -> 49.5, 512 + 32 over 6000 / 400 133 -> 78, 79-90 rows of 6
+// over 11-1469 40.1 -> 23.8. The host has the largest of each only, so several
+// sequences split up to a 128-row tile per four CUs, and per two over 512 keys
+// (396 ragged batches: 4 more than 5 % slower than unsplit, by 25 % at most).
 // Head dim 128, the decoder's, at 16- and 32-token blocks, is what is built: a
 // 16-bit cache's two stages of four tiles do not fit the LDS at head dims 192
 // and 256 (192 and 256 KiB); 64 and 96, 8-token blocks and the larger head
@@ -68,9 +75,10 @@ bool prefill_split_keys(const PrefillArgs& a, const CacheGeom& g) {
                           a.k_scale == nullptr;
     return a.max_kv_len > (!few_rows ? 2 : 4 * tiles <= cus ? 6 : 12) * kPrefillKeys;
   }
-  if (any_group)
-    return 2 * prefill_row_tiles(a.max_query_len, group, kPrefillWaves * 32) * pairs <= cus &&
-           a.max_kv_len >= 16 * kPrefillKeys;
+  const int64_t big_tiles = prefill_row_tiles(a.max_query_len, group, kPrefillWaves * 32) * pairs;
+  if (a.num_seqs > 1 && 4 * big_tiles <= cus) return a.max_kv_len > 2 * kPrefillKeys;
+  if (a.num_seqs > 1 || any_group)
+    return 2 * big_tiles <= cus && a.max_kv_len >= 16 * kPrefillKeys;
   return tiles <= 2 * cus && a.causal && a.max_query_len > 512 &&
          a.max_kv_len < 4 * (int64_t)a.max_query_len;
 }
